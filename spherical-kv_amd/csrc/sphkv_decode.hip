@@ -23,8 +23,9 @@
 //
 // Per page (16 tokens, positions pos_t), lane l = (token t = l % 16, quarter
 // u = l / 16), page centre t_mid = (min pos + max pos) / 2:
-//   1. the query rows are rotated once per page by -t_mid (fp32, lanes = RoPE
-//      frequencies j) and kept in LDS in the QK MFMA's operand order;
+//   1. the query rows are rotated once per page by -t_mid in registers (fp32):
+//      each lane holds one head slot's values on a fourth of its quarter's
+//      pairs, which is the QK MFMA's A operand as it stands (qk_mfma);
 //   2. k_hat of token t on this lane's 32 dimensions (chunk_dim):
 //      compressed  k_hat_d = r_hat_g * centroid_g[code][d mod g],
 //                  r_hat_g = int8 / 127 * scale_g         (pagebuilder.py:17-21)
@@ -290,12 +291,14 @@ __device__ __forceinline__ void load_dense(const Res& rs, const LaneOff& lo, int
   }
 }
 
-// Waves per decode workgroup: 12 (3 per SIMD, up to 168 VGPRs each), enough
-// to keep the per-lane offsets and addresses of the page loop in registers;
-// 8 (2 per SIMD, 256 VGPRs) for GQA 8, whose two head sets double the QK
-// operands and accumulators.
-template <int GQA>
-__host__ __device__ constexpr int decode_waves() { return GQA <= 4 ? 12 : 8; }
+// Waves per decode workgroup: 12 (3 per SIMD, up to 168 VGPRs each).  Waves
+// per SIMD are what hides a page's chain of LDS, phasor and MFMA latencies:
+// GQA 8 took 8 waves while its rotated queries lay in LDS (26 KB more per
+// workgroup and 16 reads of 16 bytes per lane and page); with them in
+// registers 12 fit, and 4 x 131K tokens at dh 128 went from 317 to 284 us.
+// 16 waves (128 VGPRs) spill at dh 128; 6 waves and half the LDS do not pair
+// up on a CU (34 against 23 us at 32K tokens).
+constexpr int kDecodeWaves = 12;
 constexpr int kDelta = 96;             // delta-phasor table rows: |pos - page centre| < kDelta
 
 __host__ __device__ constexpr int align16(int x) { return (x + 15) & ~15; }
@@ -308,14 +311,13 @@ __host__ __device__ constexpr int align16(int x) { return (x + 15) & ~15; }
 //    rows padded by 16 bytes;
 //  * f_j in turns per token (fp64);
 //  * per wave: the staging area of its page (1 KB: the 512-byte window, and
-//    room for the reads of tokens past the page's count), the query rows
-//    rotated to the page centre (fp32, in the QK MFMA's operand order; slots
-//    of heads >= GQA stay zero), and the page's softmax weights P as fp16
-//    [max(GQA, 4)][16 tokens] (rows >= GQA stay zero), read back as the PV
-//    MFMA's A operand.
+//    room for the reads of tokens past the page's count) and the page's
+//    softmax weights P as fp16 [max(GQA, 4)][16 tokens] (rows >= GQA stay
+//    zero), read back as the PV MFMA's A operand (pv_mfma);
+//  * the item's query rows (fp16, rows padded by 16 bytes).
 template <int DH, int GQA>
 struct DecodeLds {
-  static constexpr int kWaves = decode_waves<GQA>();
+  static constexpr int kWaves = kDecodeWaves;
   static constexpr int NJ = DH / 2;
   static constexpr int NPAIR = DH / 8;          // RoPE pairs (j, j + DH/2) per lane
   static constexpr int MQ = NPAIR / 4;          // float4 groups of pairs per lane
@@ -334,18 +336,10 @@ struct DecodeLds {
   static constexpr int stage_bytes = 1024;
   static constexpr int PR = GQA < 4 ? 4 : GQA;                   // heads padded to 4 (slots)
   static constexpr int NHS = PR / 4;                             // sets of 4 head slots
-  // rotated query, fp32, per set of 4 head slots: block (half hf, group m)
-  // of 68 floats = [quarter u][slot][4 pairs e] + 4 padding floats, the
-  // float4 of (u, slot) holding pairs 4m .. 4m + 3 of quarter u's RoPE
-  // frequencies, first (hf = 0) or second (hf = 1) half.  The A-operand
-  // reads (16 float4s of one block) and the per-frequency writes (one float
-  // per lane, banks (4 m + e + 16 u) mod 64 distinct) are conflict-free.
-  static constexpr int kQBlk = 68;
-  static constexpr int qset = 2 * MQ * kQBlk;                    // floats per head-slot set
-  static constexpr int o_qr = o_stage + kWaves * stage_bytes;
-  static constexpr int qr_wave = NHS * qset * 4;                 // bytes per wave
-  static constexpr int o_pt = o_qr + kWaves * qr_wave;
-  static constexpr int total = o_pt + kWaves * PR * 32;
+  static constexpr int o_pt = o_stage + kWaves * stage_bytes;
+  static constexpr int o_q = o_pt + kWaves * PR * 32;            // the item's query rows, fp16
+  static constexpr int q_row = DH * 2 + 16;                      // bytes per padded row
+  static constexpr int total = o_q + GQA * q_row;
   // the end-of-item wave merge reuses the space: [kWaves][GQA][DH] acc,
   // [kWaves][GQA][2] (m, l)
   static constexpr int merge_bytes = kWaves * GQA * (DH + 2) * 4;
@@ -440,6 +434,43 @@ __device__ __forceinline__ float quarter_sum(floatx4 s) {
 __host__ __device__ constexpr int row_slot(int row) { return (0xD8 >> (2 * row)) & 3; }   // {0, 2, 1, 3}
 __host__ __device__ constexpr int slot_row(int slot) { return (0xD8 >> (2 * slot)) & 3; }  // its inverse
 
+// Value of lane M of each quad (4 consecutive lanes), in all its lanes (DPP quad_perm).
+template <int M>
+__device__ __forceinline__ float quad_bcast(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x55 * M, 0xF, 0xF, true));
+}
+
+// Query pairs 4 M + b of a lane (b = lane >> 2 & 3) rotated to the page centre
+// by the phasor that lane M of its quad formed.
+template <int M, int NHS, int MQ>
+__device__ __forceinline__ void rotate_q(float2 z, const float (&qf)[NHS][MQ][2], float (&qc)[NHS][MQ][2]) {
+  const float zx = quad_bcast<M>(z.x), zy = quad_bcast<M>(z.y);
+#pragma unroll
+  for (int hs = 0; hs < NHS; ++hs) {
+    qc[hs][M][0] = qf[hs][M][0] * zx + qf[hs][M][1] * zy;
+    qc[hs][M][1] = qf[hs][M][1] * zx - qf[hs][M][0] * zy;
+  }
+}
+
+// The 4x4x1 QK products of pair 4 m + E.  The four blocks of a lane quarter
+// take their A operand from the quarter's block E (cbsz 2, abid E), so one
+// register holds four pairs' query values: block b of a quarter holds pair
+// 4 m + b, and no lane repeats another's.  (Through LDS the rotated queries
+// cost 8 writes and, per head set, 8 reads of 16 bytes per lane and page:
+// 39 LDS instructions per page against 23.)
+template <int E>
+__device__ __forceinline__ void qk_mfma(const float (&qc)[2], float x0, float x1, floatx4 (&qk)[2]) {
+  qk[0] = __builtin_amdgcn_mfma_f32_4x4x1f32(qc[0], x0, qk[0], 2, E, 0);
+  qk[1] = __builtin_amdgcn_mfma_f32_4x4x1f32(qc[1], x1, qk[1], 2, E, 0);
+}
+
+// The 4x4x4 PV product of tokens 4 TG .. 4 TG + 3: block TG of each quarter
+// holds their weights (cbsz 2, abid TG).
+template <int TG>
+__device__ __forceinline__ floatx4 pv_mfma(half4 pa, half4 vb, floatx4 acc) {
+  return __builtin_amdgcn_mfma_f32_4x4x4f16(pa, vb, acc, 2, TG, 0);
+}
+
 __device__ __forceinline__ void set_prio(int lvl) {
   if (lvl >= 3) __builtin_amdgcn_s_setprio(3);
   else if (lvl == 2) __builtin_amdgcn_s_setprio(2);
@@ -501,17 +532,17 @@ __device__ __forceinline__ void encode_new_token(float (&x)[32], const float* cr
 
 
 template <int DH, int GQA>
-__global__ __launch_bounds__(decode_waves<GQA>() * 64)
-__attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() / 4))) void decode_kernel(
+__global__ __launch_bounds__(kDecodeWaves * 64)
+__attribute__((amdgpu_waves_per_eu(kDecodeWaves / 4, kDecodeWaves / 4))) void decode_kernel(
     const int32_t* __restrict__ work, int32_t num_items, DecodeArgs a) {
   // work and num_items lead the argument list: the build preloads the first
   // kernel-argument dwords into SGPRs, so the work item's load is issued at
   // wave start instead of after two dependent argument loads
-  constexpr int kWaves = decode_waves<GQA>();
+  constexpr int kWaves = kDecodeWaves;
   constexpr int NC = DH / 32;        // 8-dim chunks of dense K per lane-token
   constexpr int NJ = DH / 2;         // RoPE frequencies
   using L = DecodeLds<DH, GQA>;
-  constexpr int NPAIR = L::NPAIR, MQ = L::MQ;
+  constexpr int NPAIR = L::NPAIR, MQ = L::MQ, NHS = L::NHS;
   __shared__ __attribute__((aligned(16))) uint8_t smem[L::total];
   float* cb_s = reinterpret_cast<float*>(smem + L::o_cb);
   const uint8_t* dtab = smem + L::o_dtab;
@@ -541,7 +572,6 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
   const int t = lane & 15;
   const int u = lane >> 4;
   uint8_t* st = smem + L::o_stage + wave * L::stage_bytes;
-  float* qr = reinterpret_cast<float*>(smem + L::o_qr + wave * L::qr_wave);
   _Float16* pt = reinterpret_cast<_Float16*>(smem + L::o_pt) + wave * L::PR * kTile;
   const LaneOff lo = lane_offsets<DH>(lane);
 
@@ -570,16 +600,15 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
       }
     }
   }
-  // this lane's query pair (j, j + NJ) of every head of the item, fp32
-  float qf[GQA][2];
-  {
-    const _Float16* qh = a.q + ((int64_t)seq * a.num_kv * GQA + (int64_t)h * GQA) * DH;
-    const int j = lane % NJ;
+  // the item's query rows, through LDS to the lanes (2-byte loads: q may have
+  // any alignment)
+  constexpr int kq = (GQA * DH + kT - 1) / kT;
+  _Float16 qv[kq];
+  const _Float16* qh = a.q + ((int64_t)seq * a.num_kv * GQA + (int64_t)h * GQA) * DH;
 #pragma unroll
-    for (int hh = 0; hh < GQA; ++hh) {
-      qf[hh][0] = (float)qh[hh * DH + j];
-      qf[hh][1] = (float)qh[hh * DH + j + NJ];
-    }
+  for (int k = 0; k < kq; ++k) {
+    const int i = threadIdx.x + k * kT;
+    qv[k] = qh[i < GQA * DH ? i : 0];
   }
   // This lane's RoPE frequency f_j (j = lane mod NJ) in turns per token.  A
   // workgroup has a multiple of NJ threads, so the delta-table entries
@@ -587,7 +616,7 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
   // table is built from registers while the first loads are in flight.
   const double f_lane = exp2(-(2.0 * (lane % NJ) / DH) * a.log2_theta) * kInvTwoPi;  // / (2 pi)
   static_assert((kWaves * 64) % NJ == 0, "delta-table rows need whole frequency runs per thread");
-  if (wave == 0 && lane < NJ) ftab[lane] = f_lane;       // the far pages' phasors read it
+  if (wave == 0 && lane < NJ) ftab[lane] = f_lane;       // the page centres' and far pages' phasors read it
   for (int i = threadIdx.x; i < kDelta * NJ; i += kT) {
     const int d = i / NJ, j = i % NJ;
     const float2 z = turn_phasor((double)d * f_lane);
@@ -613,14 +642,12 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
     if (db != kOOB) load_dense<DH>(rs, lo, db, kd);
   }
   if (GQA < 4) {
-    // zero P rows GQA..3 and the query slots GQA..3 of this wave (never written)
+    // zero P rows GQA..3 of this wave (never written)
     if (lane < (4 - GQA) * 2) {
       half8 z;
       for (int e = 0; e < 8; ++e) z[e] = (_Float16)0.f;
       *reinterpret_cast<half8*>(pt + GQA * kTile + 8 * lane) = z;
     }
-    for (int i = lane; i < 2 * MQ * 16; i += 64)          // i = (block, u, slot)
-      if ((i & 3) >= GQA) *reinterpret_cast<floatx4*>(qr + (i >> 4) * L::kQBlk + 4 * (i & 15)) = (floatx4){0.f, 0.f, 0.f, 0.f};
   }
   {
     int slot = 0;
@@ -638,26 +665,44 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
       }
     }
   }
+#pragma unroll
+  for (int k = 0; k < kq; ++k) {
+    const int i = threadIdx.x + k * kT;
+    if (i < GQA * DH) *reinterpret_cast<_Float16*>(smem + L::o_q + (i / DH) * L::q_row + 2 * (i % DH)) = qv[k];
+  }
   __syncthreads();
   // the header checks wait for this wave's header loads only (after the
   // barrier, so no wave waits for another's)
   int nbad = page_check<DH>(a, rows0, T, hdr0, 0, nwp, lane);   // malformed rows / pages of this wave
 
-  // Loop-invariant lane data: LDS addresses of this lane's query writes /
-  // reads and P write / read.
-  float* qw;
-  {
-    const int j = lane % NJ, s = j % NPAIR;
-    qw = qr + (s >> 2) * L::kQBlk + (j / NPAIR) * 16 + (s & 3);
+  // this lane's query values, fp32: head slot lane & 3 of each head set, pairs
+  // 4 m + (lane >> 2 & 3) of quarter u's RoPE pairs; slots of heads >= GQA are
+  // zero.  (Read from global memory in this order, each load touches 16 lines:
+  // 0.4 us more per work item.)
+  float qf[NHS][MQ][2];
+#pragma unroll
+  for (int hs = 0; hs < NHS; ++hs) {
+    const int hh = 4 * hs + (lane & 3);
+    const _Float16* qp = reinterpret_cast<const _Float16*>(smem + L::o_q + (hh < GQA ? hh : 0) * L::q_row) + NPAIR * u +
+                         ((lane >> 2) & 3);
+#pragma unroll
+    for (int m = 0; m < MQ; ++m) {
+      const float a0 = (float)qp[4 * m], a1 = (float)qp[4 * m + NJ];
+      qf[hs][m][0] = hh < GQA ? a0 : 0.f;
+      qf[hs][m][1] = hh < GQA ? a1 : 0.f;
+    }
   }
-  const float* qb = qr + u * 16 + (lane & 3) * 4;
+  // frequency of the page-centre phasor this lane forms: pair 4 (lane & 3) +
+  // (lane >> 2 & 3) of its quarter (DH 64: lanes with bit 1 set repeat their
+  // neighbours')
+  const double f_mid = ftab[NPAIR * u + 4 * (lane & (MQ - 1)) + ((lane >> 2) & 3)];
 
   // Online-softmax state.  After a page's quarter sums, lane (row r, token t)
   // holds the logit of head 4 hs + row_slot(r) for token t; the running
   // reference max m_run of that head is the same in all 16 lanes of the row,
   // and l_part is this lane's share (token slot t) of the head's sum of
   // weights, reduced over the row once the item is done.
-  constexpr int NHS = L::NHS, NHF = DH / 64;
+  constexpr int NHF = DH / 64;
   const int hr = row_slot(u);
   float m_run[NHS], l_part[NHS];
 #pragma unroll
@@ -714,19 +759,21 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
     const int thr = (desc >> 8) & 1023, rdr = (desc >> 18) & 1023;   // section offsets from the page start
     const bool valid = (t < n) && (pos_c >= 0);
 
-    // ---- page centre t_mid; query rows rotated by -t_mid into LDS ---------
+    // ---- page centre t_mid; query rows rotated by -t_mid -------------------
     //      <q, R(pos) k> = <R(-t_mid) q, R(pos - t_mid) k>
+    float qc[NHS][MQ][2];                       // A operands of the QK MFMA, first / second half
     {
       const int t_lo = __builtin_amdgcn_readlane(pos_c, 0);
       const int t_hi = __builtin_amdgcn_readlane(pos_c, n > 0 ? n - 1 : 0);
       const int t_mid = (t_lo >= 0 && t_hi >= 0) ? t_lo + ((t_hi - t_lo) >> 1) : max(t_lo, 0);
-      // lane = frequency j (lanes j and j + NJ write the same values when NJ = 32)
-      const float2 z = turn_phasor((double)t_mid * f_lane);
-#pragma unroll
-      for (int hh = 0; hh < GQA; ++hh) {
-        const int o = (hh >> 2) * L::qset + (hh & 3) * 4;
-        qw[o] = qf[hh][0] * z.x + qf[hh][1] * z.y;
-        qw[o + MQ * L::kQBlk] = qf[hh][1] * z.x - qf[hh][0] * z.y;
+      // the phasors of a quad's lanes s = 0 .. MQ - 1 are those of pairs 4 s +
+      // b: broadcast within the quad, they rotate this lane's query pairs
+      const float2 z = turn_phasor((double)t_mid * f_mid);
+      rotate_q<0>(z, qf, qc);
+      rotate_q<1>(z, qf, qc);
+      if constexpr (MQ == 4) {
+        rotate_q<2>(z, qf, qc);
+        rotate_q<3>(z, qf, qc);
       }
       // offset of this lane's token from the centre
       pos_c = valid ? pos_c - t_mid : 0;
@@ -743,7 +790,6 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
       else if (tid == 2) locate_k<DH, GQA, 2>(st, thr, rdr, t, u, cofs, rh);
       else locate_k<DH, GQA, 3>(st, thr, rdr, t, u, cofs, rh);
     }
-    wave_lds_sync();
 
     // ---- QK.  k_hat = (r1 c1, r2 c2) on the lane's pairs (j, j + DH/2) (c1,
     //      c2 the centroid runs of the two codebook groups, or the dense K
@@ -801,21 +847,18 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
           pc[0] = c03.x; pc[1] = c03.y; pc[2] = c03.z; pc[3] = c03.w;
           ps[0] = s03.x; ps[1] = s03.y; ps[2] = s03.z; ps[3] = s03.w;
         }
-        floatx4 q0[NHS], q1[NHS];
-#pragma unroll
-        for (int hs = 0; hs < NHS; ++hs) {
-          q0[hs] = *reinterpret_cast<const floatx4*>(qb + hs * L::qset + m * L::kQBlk);
-          q1[hs] = *reinterpret_cast<const floatx4*>(qb + hs * L::qset + (MQ + m) * L::kQBlk);
-        }
+        float x0[4], x1[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const float x0 = k1[e] * pc[e] - k2[e] * ps[e];
-          const float x1 = k2[e] * pc[e] + k1[e] * ps[e];
+          x0[e] = k1[e] * pc[e] - k2[e] * ps[e];
+          x1[e] = k2[e] * pc[e] + k1[e] * ps[e];
+        }
 #pragma unroll
-          for (int hs = 0; hs < NHS; ++hs) {
-            qk[hs][0] = __builtin_amdgcn_mfma_f32_4x4x1f32(q0[hs][e], x0, qk[hs][0], 0, 0, 0);
-            qk[hs][1] = __builtin_amdgcn_mfma_f32_4x4x1f32(q1[hs][e], x1, qk[hs][1], 0, 0, 0);
-          }
+        for (int hs = 0; hs < NHS; ++hs) {
+          qk_mfma<0>(qc[hs][m], x0[0], x1[0], qk[hs]);
+          qk_mfma<1>(qc[hs][m], x0[1], x1[1], qk[hs]);
+          qk_mfma<2>(qc[hs][m], x0[2], x1[2], qk[hs]);
+          qk_mfma<3>(qc[hs][m], x0[3], x1[3], qk[hs]);
         }
       }
     };
@@ -891,18 +934,14 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
     wave_lds_sync();
 #pragma unroll
     for (int hs = 0; hs < NHS; ++hs) {
-      const half8* prow = reinterpret_cast<const half8*>(pt + (4 * hs + (lane & 3)) * kTile);
-      const half8 p0 = prow[0], p1 = prow[1];
+      const half4 pa = *reinterpret_cast<const half4*>(pt + (4 * hs + (lane & 3)) * kTile + (lane & 12));
 #pragma unroll
-      for (int tg = 0; tg < 4; ++tg) {
-        const half8 pp = tg < 2 ? p0 : p1;
-        const half4 pa4 = (tg & 1) ? half4{pp[4], pp[5], pp[6], pp[7]} : half4{pp[0], pp[1], pp[2], pp[3]};
-#pragma unroll
-        for (int hf = 0; hf < NHF; ++hf) {
-          const half8 vv = vreg[2 * hf + (tg >> 1)];
-          const half4 vb = (tg & 1) ? half4{vv[4], vv[5], vv[6], vv[7]} : half4{vv[0], vv[1], vv[2], vv[3]};
-          acc[hs][hf] = __builtin_amdgcn_mfma_f32_4x4x4f16(pa4, vb, acc[hs][hf], 0, 0, 0);
-        }
+      for (int hf = 0; hf < NHF; ++hf) {
+        const half8 v0 = vreg[2 * hf], v1 = vreg[2 * hf + 1];
+        acc[hs][hf] = pv_mfma<0>(pa, half4{v0[0], v0[1], v0[2], v0[3]}, acc[hs][hf]);
+        acc[hs][hf] = pv_mfma<1>(pa, half4{v0[4], v0[5], v0[6], v0[7]}, acc[hs][hf]);
+        acc[hs][hf] = pv_mfma<2>(pa, half4{v1[0], v1[1], v1[2], v1[3]}, acc[hs][hf]);
+        acc[hs][hf] = pv_mfma<3>(pa, half4{v1[4], v1[5], v1[6], v1[7]}, acc[hs][hf]);
       }
     }
 
@@ -919,11 +958,17 @@ __attribute__((amdgpu_waves_per_eu(decode_waves<GQA>() / 4, decode_waves<GQA>() 
     }
     wave_lds_sync();
   };
-  for (int k = 0; k < nwp; k += 2) {
+  // Whole pairs, then the last page of an odd count.  Left between its halves,
+  // the loop got one latch for leaving and repeating; along it the second
+  // half's V loads look unconsumed at the loop's head, and the compiler waited
+  // there for the first half's V before its K path (8 heads per kv head, 4 x 131K tokens: 295
+  // against 284 us per step; 64 x U[2K, 32K]: 528 against 516).
+  int k = 0;
+  for (; k + 2 <= nwp; k += 2) {
     step(k, stg_c, pos_c, stg_b, pos_b);
-    if (k + 1 >= nwp) break;
     step(k + 1, stg_b, pos_b, stg_c, pos_c);
   }
+  if (k < nwp) step(k, stg_c, pos_c, stg_b, pos_b);
 
   __builtin_amdgcn_s_setprio(0);
   if (nbad != 0 && lane == 0) __hip_atomic_fetch_add(a.status, (uint32_t)nbad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1560,7 +1605,7 @@ static int launch_decode_t(const DecodeLaunch& L, int phases, hipStream_t stream
   const DecodeArgs a = decode_args<DH, GQA>(L);
   if (L.num_items > 0) {
     if (phases & kPhasePartials)
-      launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(decode_waves<GQA>() * 64), stream, L.work,
+      launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(kDecodeWaves * 64), stream, L.work,
                    L.num_items, a);
     const int nsh = L.num_seqs * L.num_kv;
     if ((phases & kPhaseMerge) && nsh > 0)
@@ -1591,7 +1636,7 @@ static int launch_decode_tail_t(const DecodeLaunch& L, const TailLaunch& T, hipS
   t.mode = T.mode; t.num_items = L.num_items; t.num_rows = L.num_rows; t.parity = T.parity & 1;
   const int nsh = L.num_seqs * L.num_kv;
   if ((T.mode & kTailDecode) && L.num_items > 0)
-    launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(decode_waves<GQA>() * 64), stream, L.work,
+    launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(kDecodeWaves * 64), stream, L.work,
                  L.num_items, a);
   constexpr int NSL = (GQA * DH) / (GQA * DH < 128 ? GQA * DH : 128);
   if (nsh > 0)

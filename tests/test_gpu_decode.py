@@ -547,3 +547,18 @@ def test_decode_runner_equals_decode_paged(gpu, config, ctx):
     fn2(q.data_ptr(), d.data_ptr())
     torch.cuda.synchronize()
     assert torch.equal(a, d)
+
+
+@pytest.mark.parametrize("config,gqa", [(1, 4), (1, 8), (2, 1), (2, 2), (2, 4), (5, 8)])
+@pytest.mark.parametrize("rpi", [1, 11, 13, 24, 37])
+def test_decode_pages_per_wave_edges(gpu, config, gqa, rpi):
+    # 12 waves per item: items that leave waves without a page, and waves with
+    # one page, an odd and an even count (the page loop runs whole pairs, then
+    # the last page), at every head-slot layout of the QK operand
+    wl = synth.make_decode_workload(config, ctx_override=1300, **({"num_seqs_override": 1} if config == 5 else {}))
+    wl.gqa, wl.q = gqa, np.random.default_rng(gqa).standard_normal((1, wl.num_kv * gqa, wl.dh)).astype(np.float16)
+    log(f"pages per wave: config{config} gqa={gqa} rows per item {rpi}")
+    pool, cpu = pool_from_oracle(wl, gpu, rows_per_item=rpi)
+    got = _decode(pool, wl, gpu)
+    want = oracle.decode_mode_b(cpu, wl.plan, wl.codebooks, wl.q, wl.gqa, wl.rope_theta)
+    assert max_err(got, want) <= TOL
