@@ -1160,11 +1160,23 @@ struct TailArgs {
 };
 
 constexpr int kTailThreads = 256;
+constexpr int kTailNarrowMax = 512;      // most workgroups of the narrow form (two per CU)
 
-template <int DH, int GQA>
+// Output floats of one tail workgroup: 128, or (wide) up to 512.  Each
+// workgroup of a (seq, head) repeats its loads, the new token's encode and the
+// tail's phasors, which is the shortest chain while all of them are resident
+// (3 per CU: 132 VGPRs).  With more the narrow form runs in rounds: 512 (seq,
+// head)s of 4 slices took 15.8 us, as 512 wide workgroups 7; 192 of them 41.6
+// us per step against 40.8 wide, 128 the same either way.
+__host__ __device__ constexpr int tail_slice(int dh, int gqa, bool wide) {
+  const int n = dh * gqa, most = wide ? 512 : 128;
+  return n < most ? n : most;
+}
+
+template <int DH, int GQA, bool WIDE>
 __global__ __launch_bounds__(kTailThreads) void decode_tail_kernel(DecodeArgs a, TailArgs t) {
   constexpr int G3 = DH / 32, NJ = DH / 2, NS = kTailSlots;
-  constexpr int SL = GQA * DH < 128 ? GQA * DH : 128;  // output floats of one workgroup (a slice)
+  constexpr int SL = tail_slice(DH, GQA, WIDE);        // output floats of one workgroup (a slice)
   constexpr int NSL = (GQA * DH) / SL;                 // slices per (seq, head)
   constexpr int HPS = SL / DH;                         // q heads per slice
   constexpr int COLS = SL / 4;                         // float4 columns of a slice
@@ -1638,9 +1650,11 @@ static int launch_decode_tail_t(const DecodeLaunch& L, const TailLaunch& T, hipS
   if ((T.mode & kTailDecode) && L.num_items > 0)
     launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(kDecodeWaves * 64), stream, L.work,
                  L.num_items, a);
-  constexpr int NSL = (GQA * DH) / (GQA * DH < 128 ? GQA * DH : 128);
-  if (nsh > 0)
-    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA>), dim3(nsh * NSL), dim3(kTailThreads), 0, stream, a, t);
+  constexpr int NSL = (GQA * DH) / tail_slice(DH, GQA, false), NSW = (GQA * DH) / tail_slice(DH, GQA, true);
+  if (nsh * NSL > kTailNarrowMax)
+    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, true>), dim3(nsh * NSW), dim3(kTailThreads), 0, stream, a, t);
+  else if (nsh > 0)
+    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, false>), dim3(nsh * NSL), dim3(kTailThreads), 0, stream, a, t);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -276,3 +276,34 @@ def test_second_tail_on_a_pool_is_refused(gpu):
     wl, st, pool, cpu, tail, orc = _setup(gpu, config=1, ctx=256, steps=1, capacity=1)
     with pytest.raises(ValueError, match="already has a DecodeTail"):
         ops.DecodeTail(pool, wl.gqa, wl.rope_theta, capacity=1)
+
+
+@pytest.mark.parametrize("config,seqs,rpi", [(4, 17, None), (4, 17, 1), (5, 9, None)])
+def test_decode_step_wide_slices_match_oracle(gpu, config, seqs, rpi):
+    # more (seq, head) slices than two workgroups per CU: the tail kernel's
+    # wide form (512 output floats per workgroup), with one item per (seq,
+    # head) and with more items than one round trip of its item lanes; steps
+    # before, at and after a flush
+    steps = 18
+    wl = synth.make_decode_workload(config, ctx_override=200, num_seqs_override=seqs)
+    st = synth.make_tail_steps(wl, steps)
+    wl.codebooks[3] = st.cb3
+    pool, cpu = pool_from_oracle(wl, gpu)
+    tail = ops.DecodeTail(pool, wl.gqa, wl.rope_theta, capacity=2, rows_per_item=rpi)
+    orc = TailOracle(wl.num_seqs, wl.num_kv, wl.dh, st.cb3)
+    assert wl.num_seqs * wl.num_kv * wl.gqa * wl.dh > 512 * 128
+    log(f"wide tail: config{config} seqs={seqs} items={tail.num_items}")
+    for t in range(steps):
+        q, k, v, p = st.q[t], st.k[t], st.v[t], st.pos[t]
+        out = ops.decode_step(pool, tail, _dev(q, gpu), _dev(k, gpu), _dev(v, gpu), _dev(p, gpu))
+        if t in (0, 1, 15, 17):
+            want = oracle.decode_mode_b(cpu, wl.plan, wl.codebooks, q, wl.gqa, wl.rope_theta, tail=orc,
+                                        k_new=k, v_new=v, cur_pos=p)
+            err = max_err(out.float().cpu().numpy(), want)
+            log(f"  step {t}: max abs err {err:.3e}")
+            assert err <= TOL
+        for s in range(wl.num_seqs):
+            for h in range(wl.num_kv):
+                orc.append(s, h, k[s, h], v[s, h], int(p[s]))
+    torch.cuda.synchronize()
+    _check_state(wl, pool, tail, orc)
