@@ -115,3 +115,26 @@ def test_work_helpers_reject_bad_row_starts():
         ops.make_work(np.array([0, 2 ** 31]), 8)
     work, ws = ops.make_work(np.array([3]), 8)                 # no ranges
     assert work.shape == (0, 4) and list(ws) == [0]
+
+
+@pytest.mark.parametrize("lens,want", [
+    ([2049] * 8, 65),                        # one item per CU, as before
+    ([0] * 8, 8),
+    ([36] * 1024, 64),                       # more ranges than three rounds: one item each
+    ([20] * 512, 64),
+    ([2000] * 512, 1000),                    # long contexts: about four items per CU
+])
+def test_pool_rows_per_item_regimes(lens, want):
+    rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    assert ops.pool_rows_per_item(rs, 256) == want
+
+
+@pytest.mark.parametrize("num_sh", [100, 208, 256, 257, 512, 768, 769])
+def test_pool_rows_per_item_is_bounded(num_sh):
+    # never more items than three per CU and one per range, or the one-item
+    # rule's own count
+    rng = np.random.default_rng(num_sh)
+    lens = rng.integers(10, 1000, size=num_sh) * (rng.random(num_sh) < 0.9)
+    rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    n, n1 = (_items(lens, f(rs, 256)) for f in (ops.pool_rows_per_item, ops.auto_rows_per_item))
+    assert n <= max(768, num_sh, n1)
