@@ -1,9 +1,11 @@
 // Fused encode + bitpack + page build + V placement (gfx950).
 //
-// One 8-wave workgroup per four consecutive pages: one lane per token, one
-// wave per group in the nearest-centroid phase, then one wave per page for
-// the page build and one per page for its V placement.  Per (token, group)
-// the radius, direction and code reproduce torch CPU's operation order of
+// One 8-wave workgroup per four consecutive pages (eight at dh 64); a wave's
+// lanes are the 64 tokens of four pages and the wave takes 16 of their
+// dimensions: it places those dimensions of V (and of dense pages' K), and
+// encodes the codebook group they form (32 dimensions, in half of the waves,
+// at tier 3).  Then one wave per page packs it.  Per (token, group) the radius
+// and code reproduce torch CPU's operation order of
 // _encode_keys_with_codebooks (spherical_kv_pipeline.py:1136-1144) bit for
 // bit:
 //   r    = sqrtf(sum over 8 lanes of fmaf(x, x, .) chains, lanes summed in order)
@@ -11,14 +13,14 @@
 //   code = first index of the maximum similarity, where the similarity is
 //          scored in the order of the torch path the page's size selects
 //          (code_sim / code_sim_m1 below).
-// The g = 16 tiers (1, 2) first rank all codes on v_mfma_f32_16x16x16_f16
-// with fp16 copies of the direction and the codebook rows (LDS); only the
-// codes within a proven error bound of the approximate maximum are then scored
-// exactly.  The g = 32 tier (3) scores every code exactly with the codebook
-// rows as scalar operands.  The page of pagebuilder.py:8-33 (header, fp32
-// scales, LSB-first theta codes, int8 radius codes) is built in LDS and
-// stored.  This file is compiled with -ffp-contract=off so no multiply/add
-// pair is fused except where fmaf is written.
+// The codes are found on MFMA from the keys themselves and the codebook rows
+// as two fp16 terms: wherever the best approximate similarity leads the second
+// by more than the proven error of both, it is the exact maximum; the others
+// (about one token-group in 2,000 for random keys) are scored exactly.  The
+// page of pagebuilder.py:8-33 (header, fp32 scales, LSB-first theta codes,
+// int8 radius codes) is built in LDS and stored.  This file is compiled with
+// -ffp-contract=off so no multiply/add pair is fused except where fmaf is
+// written.
 #include "sphkv_common.h"
 #include "sphkv_internal.h"
 
@@ -48,75 +50,57 @@ struct EncodeArgs {
   int32_t codes_only;       // 1: write r_out / code_out only (no pages, no V)
 };
 
-template <int DH>
-__device__ __forceinline__ void load_group(const EncodeArgs& a, int64_t row, int col0, int g, float* x) {
-  if (a.k_is_fp32) {
-    const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(a.k) + row * DH + col0);
-    for (int i = 0; i < g / 4; ++i) {
-      float4 v4 = src[i];
-      x[4 * i] = v4.x; x[4 * i + 1] = v4.y; x[4 * i + 2] = v4.z; x[4 * i + 3] = v4.w;
-    }
-  } else {
-    const half8* src = reinterpret_cast<const half8*>(static_cast<const __half*>(a.k) + row * DH + col0);
-    for (int i = 0; i < g / 8; ++i) {
-      half8 h = src[i];
-      for (int j = 0; j < 8; ++j) x[8 * i + j] = (float)h[j];
-    }
-  }
-}
-
 typedef const float __attribute__((address_space(4)))* cb_ptr;   // read through the scalar cache
 
-constexpr int kEncWaves = 8;       // waves per workgroup: one per group in the argmax phase
-constexpr int kEncPages = 4;       // pages per workgroup: one lane per token of four pages
+constexpr int kEncWaves = 8;       // waves per workgroup
 constexpr int kEncMaxG = 8;        // groups per token (dh / g)
+constexpr int kSetPages = 4;       // pages of a wave: one lane per token
 
-constexpr int kCbRow = 20;         // floats per staged codebook row (16 + pad)
-
+// Pages per workgroup: dh/16 waves cover the dimensions of four pages.
 template <int DH>
+__host__ __device__ constexpr int enc_pages() { return kSetPages * kEncWaves / (DH / 16); }
+
+// LDS: the wave-private staging area holds, one after the other, V on its way
+// to dim-major order and the MFMA's B operand: per page 16 rows of the keys'
+// fp16 values (fp32 keys: a plane of their high halves, then one of the low
+// ones).  Rows are packed, so the operand reads of a wave are contiguous.
+template <int DH, bool K32>
 struct EncodeLds {
-  float r[kEncPages * kTile][kEncMaxG];        // radius of (token, group)
-  int32_t code[kEncPages * kTile][kEncMaxG];   // code of (token, group)
-  union {
-    struct {                                   // argmax phase, per wave (group)
-      float cb[kEncWaves][64][kCbRow];                  // the group's codebook rows (g = 16 tiers)
-      _Float16 dh[kEncWaves][kEncPages * kTile][20];    // fp16 direction, token-major (rows padded)
-    } arg;
-    struct {                                   // build phase
-      uint8_t stage[kEncPages][512];           // page images
-      _Float16 vt[kEncPages][DH * kTile];      // V pages, dim-major
-    } build;
-  } u;
+  static constexpr int GW = DH / 16;                       // waves per set of pages
+  static constexpr int wide = (K32 ? 2 : 1) * 1024;        // bytes of a page's keys, 32 dimensions a row
+  // waves w < DH/32 of a set may hold 32-dimension rows, the others 16
+  __host__ __device__ static constexpr int page_bytes(int w) { return w < DH / 32 ? wide : wide / 2; }
+  __host__ __device__ static constexpr int base(int wave) {
+    const int set = wave / GW, w = wave % GW;
+    const int per_set = kSetPages * wide * (DH / 32) * 3 / 2;
+    return set * per_set + kSetPages * (w < DH / 32 ? w * wide : (DH / 32) * wide + (w - DH / 32) * (wide / 2));
+  }
+  static constexpr int xs_bytes = kSetPages * wide * (DH / 32) * 3 / 2 * (kEncWaves / GW);
+  uint8_t xs[xs_bytes];
+  float r[enc_pages<DH>() * kTile][kEncMaxG + 1];          // radius of (token, group), rows padded
+  int32_t code[enc_pages<DH>() * kTile][kEncMaxG + 1];     // code of (token, group)
+  int32_t meta[enc_pages<DH>()][4];                        // tier, tokens, page offset
+  uint8_t stage[enc_pages<DH>()][512];                     // page images
 };
 
-// Nearest-centroid search of the g = 16 tiers in two stages, with the
-// group's codebook rows staged in LDS once per (tier, kv head) run.
-//  1. Approximate similarities of 16 tokens x 16 codes per
-//     v_mfma_f32_16x16x16_f16, from fp16 copies of the direction and the
-//     codebook rows.  Both are unit vectors, so |approx - s| <= 2^-10 from the
-//     two fp16 roundings (sum_i |d_i c_i| <= |d| |c| <= 1), plus at most
-//     16 * 2^-14 if the unit flushes fp16 denormals, plus the fp32 rounding of
-//     the chains (< 1e-5): eps < 2.1e-3, where s is the exact fp32 score.
-//  2. Every code c with approx_c >= max_approx - kCandSlack (>= 2 eps) is
-//     scored exactly (the torch-order chain below), in ascending order; the
-//     first maximum among them is the first maximum over all codes, because
-//     every code whose exact score equals the exact maximum passes the test.
-//     No candidate (NaN similarities) falls back to scoring every code.
-constexpr float kCandSlack = 5e-3f;
-// The bound above scales with |c|: it holds, inside the slack, for rows with
-// |c|^2 within kUnitTol of 1.  A staged codebook with any other row (scaled
-// or unnormalised rows: _encode_keys_with_codebooks accepts any codebook,
-// only codebook_loader.py:43-44 normalises) is scored exactly over every
-// code.
+// Gap between the two largest approximate similarities S = <x, c> (in units of
+// r = |x|) past which the largest is the exact first maximum.  |S - s r| <=
+// eps r for the exactly scored s, from: the codebook row's two fp16 terms
+// (2^-20), fp32 keys' two terms (2^-19), the fp32 sums of up to 96 products
+// (6e-6), the six low bits of S that carry the code (4e-6), the rounding of
+// the exact chain and of its direction (2.5e-6); eps < 1.6e-5 for rows with
+// |c|^2 <= 1.1.  The unit keeps fp16 denormals.  At 4e-5 about 0.06 % of the
+// token-groups of Gaussian keys are scored exactly; fp16 terms of the
+// direction alone need 5e-3, which left more than one candidate to one lane
+// of nearly every wave.
+constexpr float kGapSlack = 4e-5f;
+// The bound above scales with |c|: it holds for rows with |c|^2 within
+// kUnitTol of 1.  Against a codebook with any other row (scaled or
+// unnormalised rows: _encode_keys_with_codebooks accepts any codebook, only
+// codebook_loader.py:43-44 normalises) every code is scored exactly.
 constexpr float kUnitTol = 0.1f;
-
-// Does any staged row (lane < C: its 16 values) leave the unit-row bound?
-__device__ __forceinline__ bool rows_not_unit(const float4 (&row)[4], int lane, int C) {
-  float n2 = 0.f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) n2 += row[i].x * row[i].x + row[i].y * row[i].y + row[i].z * row[i].z + row[i].w * row[i].w;
-  return __builtin_amdgcn_ballot_w64(lane < C && !(fabsf(n2 - 1.f) <= kUnitTol)) != 0;   // NaN: not unit
-}
+constexpr int kOpenCode = 0x100;       // a code left to the exact scoring
+constexpr float kNoSim = -1e30f;       // no similarity yet (finite: its low bits carry a code too)
 
 // Nearest centroid of one (token, group) against the codebook rows cbg[c * GG ..]
 // (wave-uniform, so every centroid coordinate is a scalar operand): the fmaf
@@ -153,10 +137,12 @@ __device__ __forceinline__ float code_sim_m1(const float* d, const float* c) {
   return __fadd_rn(__fadd_rn(M[0], M[2]), __fadd_rn(M[1], M[3]));
 }
 
+constexpr int kOrderFma = 0, kOrderNaive = 1, kOrderM1 = 2;
+
 // Codes are scored in batches of NB rows (NB * GG = 64 floats, the scalar
 // registers one batch holds): scalar loads return in any order, so a batch's
 // rows are waited for together and their NB chains run side by side.
-template <int GG, bool NAIVE>
+template <int GG, int ORDER>
 __device__ __forceinline__ int argmax_codes(const float* dir, cb_ptr cbg, int C) {
   constexpr int NB = 64 / GG;
   float best_sim = 0.f;
@@ -169,7 +155,10 @@ __device__ __forceinline__ int argmax_codes(const float* dir, cb_ptr cbg, int C)
       for (int i = 0; i < GG; ++i) w[q][i] = cbg[(c + q) * GG + i];
     float sim[NB];
 #pragma unroll
-    for (int q = 0; q < NB; ++q) sim[q] = code_sim<GG, NAIVE>(dir, w[q]);
+    for (int q = 0; q < NB; ++q) {
+      if constexpr (ORDER == kOrderM1) sim[q] = code_sim_m1(dir, w[q]);
+      else sim[q] = code_sim<GG, ORDER == kOrderNaive>(dir, w[q]);
+    }
 #pragma unroll
     for (int q = 0; q < NB; ++q)
       if (c + q == 0 || sim[q] > best_sim) { best_sim = sim[q]; best = c + q; }
@@ -177,12 +166,13 @@ __device__ __forceinline__ int argmax_codes(const float* dir, cb_ptr cbg, int C)
   return best;
 }
 
-// Radius (torch_norm) and code of the group of GG values at element kofs of K.
-template <int GG>
-__device__ __forceinline__ void encode_group(const EncodeArgs& a, int64_t kofs, bool naive, cb_ptr cbg, int C,
+// Radius (torch_norm) and code of the group of GG values at element kofs of
+// K, every code scored exactly in the order of torch's call over `ord` tokens.
+template <int GG, bool K32>
+__device__ __forceinline__ void encode_group(const EncodeArgs& a, int64_t kofs, int ord, cb_ptr cbg, int C,
                                              float& r_out, int& code_out) {
   float x[GG];
-  if (a.k_is_fp32) {
+  if constexpr (K32) {
     const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(a.k) + kofs);
 #pragma unroll
     for (int i = 0; i < GG / 4; ++i) {
@@ -199,357 +189,573 @@ __device__ __forceinline__ void encode_group(const EncodeArgs& a, int64_t kofs, 
     }
   }
   const float r = torch_norm(x, GG);
-  const float den = __fadd_rn(r, 1e-8f);
   float dir[GG];
-  group_directions<GG>(x, den, !a.k_is_fp32, dir);
+  group_directions<GG>(x, __fadd_rn(r, 1e-8f), !K32, dir);
   r_out = r;
-  code_out = naive ? argmax_codes<GG, true>(dir, cbg, C) : argmax_codes<GG, false>(dir, cbg, C);
+  if (ord * GG * C < 400) code_out = argmax_codes<GG, kOrderNaive>(dir, cbg, C);   // torch's own small-bmm loop
+  else if (GG == 16 && ord == 1) code_out = argmax_codes<GG, GG == 16 ? kOrderM1 : kOrderFma>(dir, cbg, C);
+  else code_out = argmax_codes<GG, kOrderFma>(dir, cbg, C);
 }
 
-// One workgroup per four consecutive pages; lane = token (page slot j =
-// lane / 16, token t = lane % 16).  Argmax phase: wave w encodes group w of
-// every token, with the codebook of a (tier, kv head) as scalar operands; the
-// lanes whose page shares the first unhandled page's (tier, head) go
-// together, so four pages of one run take one pass.  Build phase: wave j < 4
-// builds page j in LDS (header, scales, LSB-first codes, int8 radius codes;
-// pagebuilder.py:8-33) and stores it, or copies a dense page's fp16 K rows;
-// wave 4 + j places page j's V rows dim-major.
-template <int DH>
-__global__ __launch_bounds__(kEncWaves * 64) void encode_pages_kernel(EncodeArgs a) {
-  __shared__ EncodeLds<DH> sm;
-  const int lane = threadIdx.x & 63;
-  const int wave = uniform(threadIdx.x >> 6);
-  const int p0 = blockIdx.x * kEncPages;                          // the workgroup's first page
+// The code of one token's 16-value group among the candidate codes of mask mk
+// (their rows at cb + 16 c), scored exactly in ascending order (calls over one
+// token at C = 64, whose order is code_sim_m1's, are left to encode_group).
+// quad(q) gives values 4 q .. 4 q + 3 of the group; four at a time, so that
+// the kernel's register count is not set here.
+template <bool K32, typename Q>
+__device__ __forceinline__ int score_candidates(Q quad, float r, bool naive, const float* cb, uint64_t mk) {
+  const float den = __fadd_rn(r, 1e-8f);
+  float best_sim = 0.f;
+  int best = -1;
+  while (mk) {
+    const int c = (int)__builtin_ctzll(mk);
+    mk &= mk - 1;
+    float4 w[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) w[q] = *reinterpret_cast<const float4*>(cb + 16 * c + 4 * q);
+    float sc = 0.f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      float x[4], d[4];
+      quad(q, x);
+      group_directions<4>(x, den, !K32, d);
+      const float v[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sc = naive ? __fadd_rn(sc, __fmul_rn(d[e], v[e])) : __builtin_fmaf(d[e], v[e], sc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (best < 0 || sc > best_sim) { best_sim = sc; best = c; }
+  }
+  return best;
+}
 
-  // ---- argmax phase: group `wave` of this lane's token ---------------------
-  {
-    const int j = lane >> 4, t = lane & 15;
-    const int p = p0 + j;
-    const bool p_ok = p < a.num_pages;
-    // the token's source row is loaded together with the page's metadata (its
-    // address does not depend on them) and masked by the count afterwards
-    const int64_t row_raw = p_ok ? a.src_rows[(int64_t)p * kTile + t] : -1;
-    const int tid_l = p_ok ? a.tier[p] : 0;
-    const int n_l = p_ok ? min(max(a.count[p], 0), kTile) : 0;
-    // the summation order follows torch's call over ord_l tokens: the page's
-    // own count, or the caller's N (a whole head's tokens in one call)
-    const int ord_l = p_ok ? (a.order_n ? max(a.order_n[p], 1) : n_l) : 0;
-    const int sh_l = p_ok ? a.seq_head[p] : -1;
-    const int head_l = sh_l >= 0 ? sh_l % a.num_kv : 0;
-    int64_t row = t < n_l ? row_raw : -1;
-    if (row >= a.num_src_rows) row = -1;
-    // a page is encoded only with its tier's codebook and a valid (seq, head)
-    const bool comp_l = tid_l >= 1 && tid_l <= 3 && wave < DH / tier_g(tid_l) && sh_l >= 0 &&
-                        a.cb[tid_l >= 1 && tid_l <= 3 ? tid_l : 0] != nullptr;
-    const int gi = wave;
-    // ---- g = 16 tiers (1, 2): MFMA similarities, exact scores for candidates
-    const bool m16_l = comp_l && tier_g(tid_l) == 16;
-    const uint64_t m16 = __builtin_amdgcn_ballot_w64(m16_l);
-    if (m16) {
-      const bool live = m16_l && row >= 0;
-      const int tl = lane & 15, kg = lane >> 4;
-      float (*cbs)[kCbRow] = sm.u.arg.cb[wave];
-      // codebook rows of the first g = 16 page's (tier, head), loaded before K
-      const int j0 = (int)__builtin_ctzll(m16) >> 4;
-      const int tid0 = uniform(__builtin_amdgcn_readlane(tid_l, 16 * j0));
-      const int h0 = uniform(__builtin_amdgcn_readlane(head_l, 16 * j0));
-      const int C0 = tier_C(tid0);                                  // 64 or 16
-      float4 crow[4];
-      {
-        const float* cbg = a.cb[tid0] + ((int64_t)h0 * (DH / 16) + gi) * C0 * 16;
+// hi + lo = x to 2^-20 |x|, as fp16 (both terms rounded towards zero).
+__device__ __forceinline__ void split_half4(const float (&x)[4], half4& hi, half4& lo) {
+  const auto h0 = __builtin_amdgcn_cvt_pkrtz(x[0], x[1]), h1 = __builtin_amdgcn_cvt_pkrtz(x[2], x[3]);
+  const auto l0 = __builtin_amdgcn_cvt_pkrtz(x[0] - (float)h0[0], x[1] - (float)h0[1]);
+  const auto l1 = __builtin_amdgcn_cvt_pkrtz(x[2] - (float)h1[0], x[3] - (float)h1[1]);
+  hi = half4{(_Float16)h0[0], (_Float16)h0[1], (_Float16)h1[0], (_Float16)h1[1]};
+  lo = half4{(_Float16)l0[0], (_Float16)l0[1], (_Float16)l1[0], (_Float16)l1[1]};
+}
+
+// The codebook rows of one (tier, kv head, group) as the MFMA's A operand, two
+// fp16 terms.  g = 16: block b of 16 codes, lane (tl, kg) holds dimensions 4 kg
+// .. 4 kg + 3 of code 16 b + tl.  g = 32: dimensions 8 kg .. 8 kg + 7 of code
+// tl < 8 (blocks 0 and 1; rows 8..15 are zero).  bad: a row's length leaves
+// kUnitTol.
+struct Codebook {
+  half4 hi[4], lo[4];
+  int tid, h;
+  bool bad;
+};
+
+template <int DH, bool G32>
+__device__ __forceinline__ void load_codebook(const EncodeArgs& a, int tid, int h, int w, int lane, Codebook& cb) {
+  const int tl = lane & 15, kg = lane >> 4;
+  const int C = G32 ? 8 : tier_C(tid);
+  constexpr int NB = G32 ? 2 : 4;
+  const float* c = G32 ? a.cb[3] + ((int64_t)h * (DH / 32) + w) * (8 * 32) + (tl & 7) * 32 + 8 * kg
+                       : a.cb[tid] + ((int64_t)h * (DH / 16) + w) * C * 16 + tl * 16 + 4 * kg;
+  float4 v[NB];
+  v[0] = *reinterpret_cast<const float4*>(c);
+  if constexpr (G32) {
+    v[1] = *reinterpret_cast<const float4*>(c + 4);
+  } else if (C == 64) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          crow[i] = lane < C0 ? *reinterpret_cast<const float4*>(cbg + lane * 16 + 4 * i) : float4{0.f, 0.f, 0.f, 0.f};
-      }
-      bool exact_all = rows_not_unit(crow, lane, C0);
-      // do all g = 16 pages of the workgroup use (tid0, h0)?
-      bool same = true;
+    for (int b = 1; b < 4; ++b) v[b] = *reinterpret_cast<const float4*>(c + 256 * b);
+  }
+  float n2[NB];                                          // squared length of the lane's part of each row
+  auto convert = [&](int b) __attribute__((always_inline)) {
+    float x[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
+    n2[b] = 0.f;
 #pragma unroll
-      for (int jj = 0; jj < kEncPages; ++jj)
-        if ((m16 >> (16 * jj)) & 0xFFFFull)
-          same = same && __builtin_amdgcn_readlane(tid_l, 16 * jj) == tid0 &&
-                 __builtin_amdgcn_readlane(head_l, 16 * jj) == h0;
-      float dir[16];
-      float r = 0.f;
-      {
-        float x[16];
-        if (live) {
-          const int64_t kofs = row * DH + gi * 16;
-          if (a.k_is_fp32) {
-            const float4* src = reinterpret_cast<const float4*>(static_cast<const float*>(a.k) + kofs);
+    for (int e = 0; e < 4; ++e) {
+      n2[b] = __builtin_fmaf(x[e], x[e], n2[b]);
+      if (G32) x[e] = tl < 8 ? x[e] : 0.f;
+    }
+    split_half4(x, cb.hi[b], cb.lo[b]);
+  };
+  convert(0);
+  float row2;
+  if constexpr (G32) {
+    convert(1);
+    row2 = rows_sum(n2[0] + n2[1]);
+  } else if (C == 64) {
+    convert(1);
+    convert(2);
+    convert(3);
+    // the four lane rows' parts added: each lane ends with one block's row
+    float a0 = n2[0], a1 = n2[1], b0 = n2[2], b1 = n2[3];
+    swap32(a0, a1);
+    swap32(b0, b1);
+    float c0 = a0 + a1, c1 = b0 + b1;
+    swap16(c0, c1);
+    row2 = c0 + c1;
+  } else {
+    row2 = rows_sum(n2[0]);
+  }
+  const bool bad = !(fabsf(row2 - 1.f) <= kUnitTol);
+  cb.tid = tid;
+  cb.h = h;
+  cb.bad = __builtin_amdgcn_ballot_w64(bad) != 0;
+}
+
+// fmaxf without the instruction that quiets its operands first
+__device__ __forceinline__ float max_raw(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ float min_raw(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+// Largest and second largest of a running pair (m1 >= m2) and s, whose six low
+// bits are replaced by (code bits of the caller); NaNs are passed over.
+__device__ __forceinline__ void top2(float s, int bits, float& m1, float& m2) {
+  const float k = __builtin_bit_cast(float, (__builtin_bit_cast(uint32_t, s) & ~63u) | (uint32_t)bits);
+  m2 = __builtin_amdgcn_fmed3f(m1, m2, k);
+  m1 = max_raw(m1, k);
+}
+__device__ __forceinline__ void top2_merge(float& a1, float& a2, float b1, float b2) {
+  const float lo = min_raw(a1, b1);
+  a1 = max_raw(a1, b1);
+  a2 = max_raw(lo, max_raw(a2, b2));
+}
+
+// K values of one token's GG dimensions of a wave: fp16 as loaded, or fp32.
+template <int GG, bool K32> struct KeyRegs { half8 h[GG / 8]; };
+template <int GG> struct KeyRegs<GG, true> { float f[GG]; };
+
+// The loads are unconditional, so nothing waits between them: lanes without a
+// token read 128 bytes of the caller's row table instead.
+template <int GG, bool K32>
+__device__ __forceinline__ void load_keys(const EncodeArgs& a, int64_t kofs, bool ok, const void* none,
+                                          KeyRegs<GG, K32>& k) {
+  if constexpr (K32) {
+    const float4* src = ok ? reinterpret_cast<const float4*>(static_cast<const float*>(a.k) + kofs)
+                           : static_cast<const float4*>(none);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const float4 v4 = src[i];
-              x[4 * i] = v4.x; x[4 * i + 1] = v4.y; x[4 * i + 2] = v4.z; x[4 * i + 3] = v4.w;
-            }
-          } else {
-            const half8* src = reinterpret_cast<const half8*>(static_cast<const __half*>(a.k) + kofs);
+    for (int i = 0; i < GG / 4; ++i) {
+      const float4 v4 = src[i];
+      k.f[4 * i] = v4.x; k.f[4 * i + 1] = v4.y; k.f[4 * i + 2] = v4.z; k.f[4 * i + 3] = v4.w;
+    }
+  } else {
+    const half8* src = ok ? reinterpret_cast<const half8*>(static_cast<const __half*>(a.k) + kofs)
+                          : static_cast<const half8*>(none);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-              const half8 hv = src[i];
+    for (int i = 0; i < GG / 8; ++i) k.h[i] = src[i];
+  }
+}
+
+// Similarities of 16 tokens (B, Bl: their keys' high and low halves) x the 16
+// codes of block b.
+template <bool K32>
+__device__ __forceinline__ floatx4 sims16(const Codebook& cb, int b, half4 B, half4 Bl) {
+  floatx4 D = __builtin_amdgcn_mfma_f32_16x16x16f16(cb.hi[b], B, (floatx4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+  D = __builtin_amdgcn_mfma_f32_16x16x16f16(cb.lo[b], B, D, 0, 0, 0);
+  if constexpr (K32) D = __builtin_amdgcn_mfma_f32_16x16x16f16(cb.hi[b], Bl, D, 0, 0, 0);
+  return D;
+}
+
+// What the exact scoring needs of a token, loaded again where it runs (so that
+// the usual path holds none of it in registers).
+struct TokenMeta {
+  int64_t row;
+  int tid, head, ord;
+};
+template <bool CODES>
+__device__ __forceinline__ TokenMeta reload_token(const EncodeArgs& a, int pc, int t) {
+  asm volatile("" : "+v"(pc));
+  TokenMeta m;
+  m.row = a.src_rows[(int64_t)pc * kTile + t];
+  m.tid = a.tier[pc];
+  m.head = max(a.seq_head[pc], 0) % a.num_kv;
+  // the summation order follows torch's call over ord tokens: the page's own
+  // count, or the caller's N (a whole head's tokens in one call)
+  m.ord = CODES && a.order_n ? max(a.order_n[pc], 1) : min(max(a.count[pc], 0), kTile);
+  return m;
+}
+
+// The wave's tokens of the pages in `comp` (a ballot: whole 16-lane rows) at
+// group size GG: radius and code of each live lane.  The keys go to LDS as the
+// MFMA's B operand; per page 16 tokens x 16 codes per MFMA, lane (tl, kg)
+// keeping the two largest similarities of token tl over codes 16 b + 4 kg + i;
+// the rows' pairs are then merged into the lanes that hold the tokens.
+template <int DH, int GG, bool K32>
+__device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs<GG, K32>& k, uint8_t* xs,
+                                              int PB, uint64_t comp, bool mine_l, bool live, int tid_l, int head_l,
+                                              int w, int lane, Codebook& cb, float& r, int& code) {
+  constexpr bool G32 = GG == 32;
+  constexpr int RB = 2 * GG;                             // bytes per staged row
+  const int j = lane >> 4, t = lane & 15;
+  r = 0.f;
+  uint8_t* dst = xs + PB * j + RB * t;
+  if constexpr (K32) {
+    if (live) r = torch_norm(k.f, GG);
+    // scaled to length 256 (a factor common to a token's similarities leaves
+    // their order): high and low fp16 halves
+    const float sc = 256.f * __builtin_amdgcn_rcpf(r);
+    if (mine_l) {
 #pragma unroll
-              for (int e = 0; e < 8; ++e) x[8 * i + e] = (float)hv[e];
-            }
-          }
-        } else {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) x[i] = 0.f;
-        }
-        r = live ? torch_norm(x, 16) : 0.f;
-        const float den = __fadd_rn(r, 1e-8f);
-        group_directions<16>(x, den, !a.k_is_fp32, dir);         // x = 0 (dir = +0) where not live
-      }
-      {
-        _Float16* d = sm.u.arg.dh[wave][lane];
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4)
-          *reinterpret_cast<half4*>(d + 4 * q4) = half4{(_Float16)dir[4 * q4], (_Float16)dir[4 * q4 + 1],
-                                                        (_Float16)dir[4 * q4 + 2], (_Float16)dir[4 * q4 + 3]};
-      }
-      if (lane < C0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(&cbs[lane][4 * i]) = crow[i];
-      }
-      wave_lds_sync();
-      // candidate codes of 16 tokens of page jj against the staged rows (A
-      // operands, codes 16 b + row); lane (tl, kg) ends with token tl's mask
-      auto page_masks = [&](int jj, int C, const half4 (&A)[4], uint32_t& lo, uint32_t& hi) {
-        const half4 B = *reinterpret_cast<const half4*>(sm.u.arg.dh[wave][16 * jj + tl] + 4 * kg);
-        floatx4 D[4];
-        float mloc = -INFINITY;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          if (16 * b < C) {
-            D[b] = __builtin_amdgcn_mfma_f32_16x16x16f16(A[b], B, (floatx4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mloc = fmaxf(mloc, D[b][i]);    // D[b][i]: code 16 b + 4 kg + i, token tl
-          }
-        }
-        const float thr = rows_max(mloc) - kCandSlack;
-        lo = 0u;
-        hi = 0u;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          if (16 * b < C) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              const int c = 16 * b + 4 * kg + i;
-              if (D[b][i] >= thr) {
-                if (c < 32) lo |= 1u << c;
-                else hi |= 1u << (c - 32);
-              }
-            }
-          }
-        }
-        lo = rows_or(lo);
-        hi = rows_or(hi);
-      };
-      auto load_A = [&](int C, half4 (&A)[4]) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const float4 cv = 16 * b < C ? *reinterpret_cast<const float4*>(&cbs[16 * b + tl][4 * kg]) : float4{0.f, 0.f, 0.f, 0.f};
-          A[b] = half4{(_Float16)cv.x, (_Float16)cv.y, (_Float16)cv.z, (_Float16)cv.w};
-        }
-      };
-      // exact scores of this lane's token over the codes of mask (lo, hi)
-      auto score = [&](uint32_t lo, uint32_t hi, int C) {
-        uint64_t mk = (uint64_t)lo | ((uint64_t)hi << 32);
-        if (C < 64) mk &= (1ull << C) - 1;
-        if (mk == 0 || exact_all) mk = C == 64 ? ~0ull : ((1ull << C) - 1);   // NaN similarities or
-                                                                                // non-unit rows: every code
-        const bool naive = ord_l * 16 * C < 400;                     // torch's own small-bmm loop
-        const bool m1 = !naive && ord_l == 1;                        // MKL's M = 1 kernel
-        float best_sim = 0.f;
-        int best = -1;
-        while (mk) {
-          const int c = (int)__builtin_ctzll(mk);
-          mk &= mk - 1;
-          float w[16];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float4 v4 = *reinterpret_cast<const float4*>(&cbs[c][4 * i]);
-            w[4 * i] = v4.x; w[4 * i + 1] = v4.y; w[4 * i + 2] = v4.z; w[4 * i + 3] = v4.w;
-          }
-          const float sc = naive ? code_sim<16, true>(dir, w) : (m1 ? code_sim_m1(dir, w) : code_sim<16, false>(dir, w));
-          if (best < 0 || sc > best_sim) { best_sim = sc; best = c; }
-        }
-        return best;
-      };
-      if (same) {
-        // one set of A operands and one exact pass for all four pages
-        half4 A[4];
-        load_A(C0, A);
-        uint32_t mlo = 0u, mhi = 0u;
-#pragma unroll
-        for (int jj = 0; jj < kEncPages; ++jj) {
-          if (((m16 >> (16 * jj)) & 0xFFFFull) == 0) continue;
-          uint32_t lo, hi;
-          page_masks(jj, C0, A, lo, hi);
-          if ((lane >> 4) == jj) { mlo = lo; mhi = hi; }               // lane 16 jj + t: token t of page jj
-        }
-        if (live) {
-          sm.r[lane][gi] = r;
-          sm.code[lane][gi] = score(mlo, mhi, C0);
-        }
-      } else {
-        // pages of several (tier, head) runs: one page at a time, restaging
-        int st_tid = tid0, st_h = h0;
-        for (int jj = 0; jj < kEncPages; ++jj) {
-          if (((m16 >> (16 * jj)) & 0xFFFFull) == 0) continue;
-          const int tid = uniform(__builtin_amdgcn_readlane(tid_l, 16 * jj));
-          const int h = uniform(__builtin_amdgcn_readlane(head_l, 16 * jj));
-          const int C = tier_C(tid);
-          if (tid != st_tid || h != st_h) {
-            wave_lds_sync();
-            const float* cbg = a.cb[tid] + ((int64_t)h * (DH / 16) + gi) * C * 16;
-            float4 row[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              row[i] = lane < C ? *reinterpret_cast<const float4*>(cbg + lane * 16 + 4 * i) : float4{0.f, 0.f, 0.f, 0.f};
-            if (lane < C) {
-#pragma unroll
-              for (int i = 0; i < 4; ++i) *reinterpret_cast<float4*>(&cbs[lane][4 * i]) = row[i];
-            }
-            exact_all = rows_not_unit(row, lane, C);
-            st_tid = tid;
-            st_h = h;
-            wave_lds_sync();
-          }
-          half4 A[4];
-          load_A(C, A);
-          uint32_t lo, hi;
-          page_masks(jj, C, A, lo, hi);
-          if (live && (lane >> 4) == jj) {
-            sm.r[lane][gi] = r;
-            sm.code[lane][gi] = score(lo, hi, C);
-          }
-        }
-      }
-      if (m16_l && !live) {
-        sm.r[lane][gi] = 0.f;
-        sm.code[lane][gi] = 0;
+      for (int q = 0; q < GG / 4; ++q) {
+        const float x4[4] = {k.f[4 * q] * sc, k.f[4 * q + 1] * sc, k.f[4 * q + 2] * sc, k.f[4 * q + 3] * sc};
+        half4 hi, lo;
+        split_half4(x4, hi, lo);
+        *reinterpret_cast<half4*>(dst + 8 * q) = hi;
+        *reinterpret_cast<half4*>(dst + 16 * RB + 8 * q) = lo;
       }
     }
-    // ---- other tiers (g = 32): exact scan with scalar codebook rows
-    uint64_t todo = __builtin_amdgcn_ballot_w64(comp_l && !m16_l);
-    while (todo) {
-      const int lead = (int)__builtin_ctzll(todo);                 // first lane not yet encoded
-      const int tid = uniform(__builtin_amdgcn_readlane(tid_l, lead));
-      const int h = uniform(__builtin_amdgcn_readlane(head_l, lead));
-      const bool mine = comp_l && !m16_l && tid_l == tid && head_l == h;
-      todo &= ~__builtin_amdgcn_ballot_w64(mine);
-      const int g = uniform(tier_g(tid)), C = uniform(tier_C(tid)), G = DH / g;
-      const uint64_t cba = (uint64_t)(a.cb[tid] + ((int64_t)h * G + gi) * C * g);
-      const cb_ptr cbg = (cb_ptr)(((uint64_t)(uint32_t)uniform((int)(cba >> 32)) << 32) |
-                                  (uint32_t)uniform((int)(uint32_t)cba));
-      if (mine) {
-        const bool naive = ord_l * g * C < 400;                   // torch's own small-bmm loop
-        float r = 0.f;
-        int code = 0;
-        if (row >= 0) {
-          if (g == 16) encode_group<16>(a, row * DH + gi * 16, naive, cbg, C, r, code);
-          else encode_group<32>(a, row * DH + gi * 32, naive, cbg, C, r, code);
+  } else {
+    if (mine_l) {
+#pragma unroll
+      for (int q = 0; q < GG / 8; ++q) *reinterpret_cast<half8*>(dst + 16 * q) = k.h[q];
+    }
+    float x[GG];
+#pragma unroll
+    for (int i = 0; i < GG; ++i) x[i] = (float)k.h[i / 8][i % 8];
+    if (live) r = torch_norm(x, GG);
+  }
+  wave_lds_sync();
+  float m1[kSetPages], m2[kSetPages];
+  uint32_t bad_pages = 0u;
+#pragma unroll
+  for (int jj = 0; jj < kSetPages; ++jj) {
+    m1[jj] = kNoSim;
+    m2[jj] = kNoSim;
+    if (((comp >> (16 * jj)) & 0xFFFFull) == 0) continue;
+    const int tid = G32 ? 3 : uniform(__builtin_amdgcn_readlane(tid_l, 16 * jj));
+    const int h = uniform(__builtin_amdgcn_readlane(head_l, 16 * jj));
+    if (tid != cb.tid || h != cb.h) load_codebook<DH, G32>(a, tid, h, w, lane, cb);
+    bad_pages |= (uint32_t)cb.bad << jj;
+    const uint8_t* xp = xs + PB * jj + RB * t;
+    if constexpr (G32) {
+      const half8 A0 = __builtin_shufflevector(cb.hi[0], cb.hi[1], 0, 1, 2, 3, 4, 5, 6, 7);
+      const half8 A1 = __builtin_shufflevector(cb.lo[0], cb.lo[1], 0, 1, 2, 3, 4, 5, 6, 7);
+      const half8 B = *reinterpret_cast<const half8*>(xp + 16 * j);
+      floatx4 D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, B, (floatx4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, B, D, 0, 0, 0);
+      if constexpr (K32) {
+        const half8 Bl = *reinterpret_cast<const half8*>(xp + 16 * RB + 16 * j);
+        D = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, Bl, D, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) top2(j < 2 ? D[i] : kNoSim, i, m1[jj], m2[jj]);   // rows 8..15 hold no code
+    } else {
+      const half4 B = *reinterpret_cast<const half4*>(xp + 8 * j);
+      half4 Bl{};
+      if constexpr (K32) Bl = *reinterpret_cast<const half4*>(xp + 16 * RB + 8 * j);
+      auto block = [&](int b) __attribute__((always_inline)) { return sims16<K32>(cb, b, B, Bl); };
+      if (tier_C(tid) == 64) {
+        const floatx4 D[4] = {block(0), block(1), block(2), block(3)};
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) top2(D[b][i], 16 * b + i, m1[jj], m2[jj]);
+      } else {
+        const floatx4 D = block(0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) top2(D[i], i, m1[jj], m2[jj]);
+      }
+    }
+    m1[jj] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, m1[jj]) | (uint32_t)(4 * j));
+  }
+  // two rounds of row swaps: row r ends with page r
+  float a0 = m1[0], a1 = m1[2], b0 = m1[1], b1 = m1[3];
+  float c0 = m2[0], c1 = m2[2], d0 = m2[1], d1 = m2[3];
+  swap32(a0, a1);
+  swap32(c0, c1);
+  swap32(b0, b1);
+  swap32(d0, d1);
+  top2_merge(a0, c0, a1, c1);
+  top2_merge(b0, d0, b1, d1);
+  swap16(a0, b0);
+  swap16(c0, d0);
+  top2_merge(a0, c0, b0, d0);
+  code = (int)(__builtin_bit_cast(uint32_t, a0) & 63u);
+  const float unit = K32 ? 256.f : r;
+  const bool open = live && (!(a0 - c0 > kGapSlack * unit + 1e-30f) || !(a0 > 0.1f * kNoSim) || ((bad_pages >> j) & 1u));
+  code = live ? (open ? kOpenCode : code) : 0;
+}
+
+// The wave's (token, group)s that encode_tokens left open, scored exactly.
+// Everything is loaded again, so that the usual path holds nothing for it.
+template <int DH, bool K32, bool CODES>
+__device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* xs, int PB, int pc, int w, int lane,
+                                           bool open, float& r, int& code) {
+  asm volatile("" : "+v"(lane));
+  const int j = lane >> 4, t = lane & 15;
+  const TokenMeta mt = reload_token<CODES>(a, pc, t);
+  // a gap within the slack: the page's similarities again, for the codes
+  // within it, which are then scored exactly.  (A wave in 30 comes here; a
+  // scan of all 64 codes instead held up its workgroup by 2 to 3 us.)
+#pragma unroll 1
+  for (int jj = 0; jj < kSetPages; ++jj) {
+    const int tid = uniform(__builtin_amdgcn_readlane(mt.tid, 16 * jj));
+    if (((__builtin_amdgcn_ballot_w64(open) >> (16 * jj)) & 0xFFFFull) == 0 || tid == 3) continue;
+    const int h = uniform(__builtin_amdgcn_readlane(mt.head, 16 * jj));
+    const int C = tier_C(tid);
+    Codebook cb;
+    load_codebook<DH, false>(a, tid, h, w, lane, cb);
+    if (cb.bad) continue;
+    const uint8_t* xp = xs + PB * jj + 32 * t;
+    const half4 B = *reinterpret_cast<const half4*>(xp + 8 * j);
+    half4 Bl{};
+    if constexpr (K32) Bl = *reinterpret_cast<const half4*>(xp + 512 + 8 * j);
+    const float unit = K32 ? 256.f : __shfl(r, 16 * jj + t, 64);
+    floatx4 D[4];
+    float mx = kNoSim;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (16 * b < C) {
+        D[b] = sims16<K32>(cb, b, B, Bl);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, D[b][i]);
+      }
+    const float thr = rows_max(mx) - (kGapSlack * unit + 1e-30f);
+    uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      if (16 * b < C) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) (b < 2 ? lo : hi) |= D[b][i] >= thr ? 1u << (16 * (b & 1) + i) : 0u;
+      }
+    lo = rows_or(lo << (4 * j));
+    hi = rows_or(hi << (4 * j));
+    const uint64_t mk = (uint64_t)lo | ((uint64_t)hi << 32);
+    const bool naive = mt.ord * 16 * C < 400;
+    if (open && j == jj && mk != 0 && __builtin_popcountll(mk) <= 8 && (naive || mt.ord > 1)) {
+      KeyRegs<16, K32> k;
+      load_keys<16, K32>(a, mt.row * DH + 16 * w, true, nullptr, k);
+      auto quad = [&](int q, float (&x)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (K32) x[e] = k.f[4 * q + e];
+          else x[e] = (float)k.h[q / 2][4 * (q & 1) + e];
         }
-        sm.r[lane][gi] = r;
-        sm.code[lane][gi] = code;
+      };
+      code = score_candidates<K32>(quad, r, naive, a.cb[tid] + ((int64_t)h * (DH / 16) + w) * C * 16, mk);
+      open = false;
+    }
+  }
+  // many ties (r = 0 among them), NaNs, non-unit rows and tier 3: every code
+  // scored, with the codebook rows as scalar operands, lanes of one (tier,
+  // head) at a time
+  uint64_t todo = __builtin_amdgcn_ballot_w64(open);
+  while (todo) {
+    const int lead = (int)__builtin_ctzll(todo);                 // first lane not yet encoded
+    const int tid = uniform(__builtin_amdgcn_readlane(mt.tid, lead));
+    const int h = uniform(__builtin_amdgcn_readlane(mt.head, lead));
+    const bool mine = open && mt.tid == tid && mt.head == h;
+    todo &= ~__builtin_amdgcn_ballot_w64(mine);
+    const int g = uniform(tier_g(tid)), C = uniform(tier_C(tid));
+    const uint64_t cba = (uint64_t)(a.cb[tid] + ((int64_t)h * (DH / g) + w) * C * g);
+    const cb_ptr cbg = (cb_ptr)(((uint64_t)(uint32_t)uniform((int)(cba >> 32)) << 32) |
+                                (uint32_t)uniform((int)(uint32_t)cba));
+    if (mine) {
+      if (g == 16) encode_group<16, K32>(a, mt.row * DH + 16 * w, mt.ord, cbg, C, r, code);
+      else encode_group<32, K32>(a, mt.row * DH + 32 * w, mt.ord, cbg, C, r, code);
+    }
+  }
+}
+
+// What bounds it: a workgroup is two round trips (page metadata; then keys, V
+// and codebook) and about 650 VALU instructions per wave, some 10 us under
+// load, so the rate is the workgroups resident: three per CU at 80 VGPRs and
+// 31 KB of LDS (fp32 keys: two).  Eight waves per SIMD (64 VGPRs) spill: 462
+// us against 315 for the 98,000-token batch below.  Measured (per launch): 16
+// prompts of 500..12,000 tokens 254 -> 186 us (3.7 TB/s of traffic), 8,192
+// tokens 26.7 -> 25, the same tokens' codes at three tiers 46.5 -> 29.
+template <int DH, bool K32, bool CODES>
+__global__ __launch_bounds__(kEncWaves * 64) __attribute__((amdgpu_waves_per_eu(6, 6))) void encode_pages_kernel(EncodeArgs a) {
+  using L = EncodeLds<DH, K32>;
+  constexpr int GW = L::GW, PG = enc_pages<DH>();
+  __shared__ __attribute__((aligned(16))) L sm;
+  const int lane = threadIdx.x & 63;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int set = wave / GW, w = wave % GW;
+  const int p0 = blockIdx.x * PG;                                  // the workgroup's first page
+  const int ps = p0 + kSetPages * set;                             // the wave's first page
+
+  // ---- this lane's token: page j, slot t; its page's metadata -------------
+  const int j = lane >> 4, t = lane & 15;
+  const int p = ps + j;
+  const bool p_ok = p < a.num_pages;
+  const int pc = p_ok ? p : a.num_pages - 1;
+  // the token's source row is loaded together with the page's metadata (its
+  // address does not depend on them) and masked by the count afterwards; no
+  // load is conditional, so they share one round trip
+  const int64_t* rows = a.src_rows + (int64_t)pc * kTile;
+  int64_t row_raw = rows[t];
+  int tid_raw = a.tier[pc], n_raw = a.count[pc], sh_raw = a.seq_head[pc];
+  int vs_l = -1, off_l = -1, th_l = -1;
+  if constexpr (!CODES) {
+    vs_l = a.vslot[pc];
+    off_l = a.ptable[3 * (int64_t)pc];
+    th_l = a.ptable[3 * (int64_t)pc + 1];
+  }
+  // (left alone, the compiler sinks loads into the branches that use them)
+  asm volatile("" : "+v"(row_raw), "+v"(tid_raw), "+v"(n_raw), "+v"(sh_raw), "+v"(vs_l), "+v"(off_l), "+v"(th_l));
+  vs_l = p_ok ? vs_l : -1;
+  const int tid_l = p_ok ? tid_raw : 0;
+  const int n_l = p_ok ? min(max(n_raw, 0), kTile) : 0;
+  const int sh_l = p_ok ? sh_raw : -1;
+  const int head_l = sh_l >= 0 ? sh_l % a.num_kv : 0;
+  const bool row_ok = t < n_l && row_raw >= 0 && row_raw < a.num_src_rows;
+  const int64_t row = row_ok ? row_raw : 0;
+  // a page is encoded only with its tier's codebook and a valid (seq, head)
+  const int have = (a.cb[1] ? 2 : 0) | (a.cb[2] ? 4 : 0) | (a.cb[3] ? 8 : 0);
+  const bool comp_l = tid_l >= 1 && tid_l <= 3 && w < DH / tier_g(tid_l) && sh_l >= 0 && ((have >> (tid_l & 3)) & 1);
+  const bool comp16_l = comp_l && tid_l != 3, comp32_l = comp_l && tid_l == 3;
+  const bool dense_l = !CODES && tid_l == kDenseTier;
+  const uint64_t comp16 = __builtin_amdgcn_ballot_w64(comp16_l), comp32 = __builtin_amdgcn_ballot_w64(comp32_l);
+  uint8_t* xs = sm.xs + L::base(wave);
+  const int PB = L::page_bytes(w);                       // bytes of a page's staged keys
+
+  // ---- K and V of the wave's dimensions, the first codebook ----------------
+  KeyRegs<16, K32> k16;
+  load_keys<16, K32>(a, row * DH + 16 * w, row_ok && (comp16_l || dense_l), rows, k16);
+  half8 vh[2];
+  if constexpr (!CODES) {
+    const half8* src = row_ok ? reinterpret_cast<const half8*>(a.v + row * DH + 16 * w) : reinterpret_cast<const half8*>(rows);
+    vh[0] = src[0];
+    vh[1] = src[1];
+  }
+  Codebook cb;
+  cb.tid = 0;
+  if (comp16) {
+    const int l0 = (int)__builtin_ctzll(comp16);
+    load_codebook<DH, false>(a, uniform(__builtin_amdgcn_readlane(tid_l, l0)), uniform(__builtin_amdgcn_readlane(head_l, l0)),
+                             w, lane, cb);
+  }
+
+  // ---- V: 64 rows of the wave's 16 dimensions through LDS; the transposing
+  //      read gives lane (i, q) tokens 4 q .. 4 q + 3 of dimension i, 8 bytes
+  //      of its dim-major row (element (token k, dim d) at d * 16 + k) --------
+  if constexpr (!CODES) {
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      uint4 d = __builtin_bit_cast(uint4, vh[k]);
+      d.x = row_ok ? d.x : 0u; d.y = row_ok ? d.y : 0u; d.z = row_ok ? d.z : 0u; d.w = row_ok ? d.w : 0u;
+      *reinterpret_cast<uint4*>(xs + 32 * lane + 16 * k) = d;
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int jj = 0; jj < kSetPages; ++jj) {
+      const int64_t vs = __builtin_amdgcn_readlane(vs_l, 16 * jj);
+      if (vs < 0 || vs >= a.num_vpages) continue;
+      typedef short short4v __attribute__((ext_vector_type(4)));
+      const uint8_t* src = xs + (16 * jj + 4 * j + (t >> 2)) * 32 + 8 * (t & 3);
+      const short4v tr = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) short4v*)src);
+      *reinterpret_cast<short4v*>(a.v_pool + (vs * DH + 16 * w + t) * kTile + 4 * j) = tr;
+    }
+    wave_lds_sync();
+  }
+
+  // ---- dense pages: header (tier id, count, six zero bytes) and fp16 K rows
+  //      at a 16-byte aligned theta offset.  A pointer-table row that does not
+  //      place the whole page inside the byte pool (negative or misaligned
+  //      offsets included) writes nothing, as a compressed page's does -------
+  if (dense_l && off_l >= 0 && (int64_t)off_l + 8 <= a.pages_bytes && (int64_t)th_l >= (int64_t)off_l + 8 &&
+      (th_l & 15) == 0 && (int64_t)th_l + (int64_t)n_l * DH * 2 <= a.pages_bytes) {
+    if (w == 0 && t < 8) a.pages[off_l + t] = t == 0 ? (uint8_t)kDenseTier : (t == 1 ? (uint8_t)n_l : 0);
+    if (t < n_l) {
+      half8* dst = reinterpret_cast<half8*>(a.pages + (int64_t)th_l + ((int64_t)t * DH + 16 * w) * 2);
+      if constexpr (K32) {
+        half8 h0, h1;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { h0[e] = (_Float16)k16.f[e]; h1[e] = (_Float16)k16.f[8 + e]; }
+        dst[0] = row_ok ? h0 : half8{};
+        dst[1] = row_ok ? h1 : half8{};
+      } else {
+        dst[0] = row_ok ? k16.h[0] : half8{};
+        dst[1] = row_ok ? k16.h[1] : half8{};
+      }
+    }
+  }
+
+  if (w == 0 && t == 0) {
+    int32_t* m = sm.meta[kSetPages * set + j];
+    m[0] = tid_l;
+    m[1] = n_l;
+    m[2] = off_l;
+  }
+
+  // ---- radii and codes ------------------------------------------------------
+  if (comp16) {
+    float r;
+    int code;
+    const bool live = comp16_l && row_ok;
+    encode_tokens<DH, 16, K32>(a, k16, xs, PB, comp16, comp16_l, live, tid_l, head_l, w, lane, cb, r, code);
+    if (comp16_l) {
+      sm.r[64 * set + lane][w] = r;
+      sm.code[64 * set + lane][w] = code;
+    }
+  }
+  if (comp32) {
+    float r;
+    int code;
+    const bool live = comp32_l && row_ok;
+    KeyRegs<32, K32> k32;
+    const int64_t row32 = reload_token<CODES>(a, pc, t).row;
+    load_keys<32, K32>(a, row32 * DH + 32 * w, live, a.src_rows + (int64_t)pc * kTile, k32);
+    const int l0 = (int)__builtin_ctzll(comp32);
+    load_codebook<DH, true>(a, 3, uniform(__builtin_amdgcn_readlane(head_l, l0)), w, lane, cb);
+    wave_lds_sync();
+    encode_tokens<DH, 32, K32>(a, k32, xs, PB, comp32, comp32_l, live, tid_l, head_l, w, lane, cb, r, code);
+    if (comp32_l) {
+      sm.r[64 * set + lane][w] = r;
+      sm.code[64 * set + lane][w] = code;
+    }
+  }
+  if (comp16 | comp32) {
+    int code = sm.code[64 * set + lane][w];
+    const bool open = (((comp16 | comp32) >> lane) & 1ull) && code == kOpenCode;
+    if (__builtin_amdgcn_ballot_w64(open)) {
+      float r = sm.r[64 * set + lane][w];
+      score_open<DH, K32, CODES>(a, xs, PB, pc, w, lane, open, r, code);
+      if (open) {
+        sm.r[64 * set + lane][w] = r;
+        sm.code[64 * set + lane][w] = code;
       }
     }
   }
   __syncthreads();
 
-  if (a.codes_only) {
+  if constexpr (CODES) {
     // radii and codes of every (token, group) of the workgroup's compressed
     // pages, [page][slot][DH / 16]
-    const int j = threadIdx.x >> 4 & 3, t = threadIdx.x & 15, gbase = threadIdx.x >> 6;
-    const int p = p0 + j;
-    if (p >= a.num_pages) return;
-    const int tid = a.tier[p];
-    if (tid < 1 || tid > 3 || t >= min(max(a.count[p], 0), kTile)) return;
-    for (int gi = gbase; gi < DH / tier_g(tid); gi += kEncWaves) {
-      const int64_t o = ((int64_t)p * kTile + t) * (DH / 16) + gi;
-      if (a.r_out) a.r_out[o] = sm.r[16 * j + t][gi];
-      if (a.code_out) a.code_out[o] = sm.code[16 * j + t][gi];
+    for (int e = threadIdx.x; e < PG * kTile * (DH / 16); e += kEncWaves * 64) {
+      const int tk = e / (DH / 16), gi = e % (DH / 16);
+      const int32_t* m = sm.meta[tk / kTile];
+      if (m[0] < 1 || m[0] > 3 || tk % kTile >= m[1] || gi >= DH / tier_g(m[0])) continue;
+      const int64_t o = (int64_t)p0 * kTile * (DH / 16) + e;
+      if (a.r_out) a.r_out[o] = sm.r[tk][gi];
+      if (a.code_out) a.code_out[o] = sm.code[tk][gi];
     }
     return;
   }
+  if (wave >= PG || p0 + wave >= a.num_pages) return;
 
-  const int j = wave & 3;
-  const int p = p0 + j;
-  if (p >= a.num_pages) return;
-  const int tid = a.tier[p];
-  const int n = min(max(a.count[p], 0), kTile);
-  const int t = lane & 15, gs = lane >> 4;
-  const bool tok_ok = t < n;
-
-  if (wave >= kEncPages) {
-    // ---- V of page j: lane (token t, quarter gs) loads DH / 4 dims of its
-    // row into LDS dim-major (element (token k, dim d) at d * 16 + k), then
-    // the wave stores whole 32-byte dim rows
-    const int64_t vs = a.vslot[p];
-    if (vs < 0 || vs >= a.num_vpages) return;
-    _Float16* vt = sm.u.build.vt[j];
-    int64_t vr = tok_ok ? a.src_rows[(int64_t)p * kTile + t] : -1;
-    if (vr >= a.num_src_rows) vr = -1;
-    constexpr int QD = DH / 4;
-#pragma unroll
-    for (int c8 = 0; c8 < QD / 8; ++c8) {
-      const int d0 = gs * QD + c8 * 8;
-      half8 hv;
-      if (vr >= 0) {
-        hv = *reinterpret_cast<const half8*>(a.v + vr * DH + d0);
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) hv[e] = (_Float16)0.f;
-      }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) vt[(d0 + e) * kTile + t] = hv[e];
-    }
-    wave_lds_sync();
-    half8* dst = reinterpret_cast<half8*>(a.v_pool + vs * DH * kTile);
-    for (int i = lane; i < DH * kTile / 8; i += kWave) dst[i] = *reinterpret_cast<const half8*>(vt + 8 * i);
-    return;
-  }
-
-  // ---- page j ---------------------------------------------------------------
-  const int64_t page_off = a.ptable[3 * p];
-  const int64_t th_off = a.ptable[3 * p + 1];
-  if (tid == kDenseTier) {
-    // header: tier id, count, six zero bytes; payload fp16 [n, DH] at a
-    // 16-byte aligned theta offset.  A pointer-table row that does not place
-    // the whole page inside the byte pool (negative or misaligned offsets
-    // included) writes nothing, as a compressed page's does.
-    if (page_off < 0 || page_off + 8 > a.pages_bytes || th_off < page_off + 8 || (th_off & 15) != 0 ||
-        th_off + (int64_t)n * DH * 2 > a.pages_bytes)
-      return;
-    if (lane < 8) a.pages[page_off + lane] = lane == 0 ? (uint8_t)kDenseTier : (lane == 1 ? (uint8_t)n : 0);
-    for (int i = lane; i < n * DH / 8; i += kWave) {
-      const int tt = i / (DH / 8), c8 = i % (DH / 8);
-      const int64_t rr = a.src_rows[(int64_t)p * kTile + tt];
-      half8 hv;
-      if (rr >= 0 && rr < a.num_src_rows) {
-        if (a.k_is_fp32) {
-          const float* src = static_cast<const float*>(a.k) + rr * DH + c8 * 8;
-          for (int e = 0; e < 8; ++e) hv[e] = (_Float16)src[e];
-        } else {
-          hv = *reinterpret_cast<const half8*>(static_cast<const __half*>(a.k) + rr * DH + c8 * 8);
-        }
-      } else {
-        for (int e = 0; e < 8; ++e) hv[e] = (_Float16)0.f;
-      }
-      *reinterpret_cast<half8*>(a.pages + th_off + ((int64_t)tt * DH + c8 * 8) * 2) = hv;
-    }
-    return;
-  }
+  // ---- page build: wave = page; lane = (token t, quarter gs) -----------------
+  const int tid = uniform(sm.meta[wave][0]), n = uniform(sm.meta[wave][1]);
+  const int64_t page_off = uniform(sm.meta[wave][2]);
+  const int64_t pg = p0 + wave;
   if (tid < 1 || tid > 3) return;
-
+  int tx = threadIdx.x;
+  asm volatile("" : "+v"(tx));                           // (formed again rather than held, and spilled, until here)
+  const int lane_b = tx & 63, tk = tx & 15, gs = lane_b >> 4;
+  const bool tok_ok = tk < n;
   const int g = tier_g(tid), b = tier_b(tid);
   const int G = DH / g;
-  const int nk = (G + 3) / 4;                   // groups per lane (2 for g=16, 1 for g=32 at DH=128)
+  const int nk = (G + 3) / 4;                   // groups per lane_b (2 for g=16, 1 for g=32 at DH=128)
   float rr_[2] = {0.f, 0.f};
   int best_[2] = {0, 0};
   for (int k = 0; k < nk; ++k) {
     const int gi = gs + 4 * k;
-    if (gi < G) { rr_[k] = sm.r[16 * j + t][gi]; best_[k] = sm.code[16 * j + t][gi]; }
+    if (gi < G) { rr_[k] = sm.r[16 * wave + tk][gi]; best_[k] = sm.code[16 * wave + tk][gi]; }
   }
   // radius scale per group: max over the page's tokens (lanes of one 16-row)
   float scale_[2];
@@ -558,28 +764,28 @@ __global__ __launch_bounds__(kEncWaves * 64) void encode_pages_kernel(EncodeArgs
     for (int o = 1; o < 16; o <<= 1) m = fmaxf(m, shfl_xor(m, o));
     scale_[k] = m;
   }
-  uint8_t* st = sm.u.build.stage[j];
+  uint8_t* st = sm.stage[wave];
   const int nG = n * G;
   const int tb = (nG * b + 7) / 8;
   const int hdr = kHeaderBytes + 4 * G;
   const int size = hdr + tb + nG;
-  if (lane < kHeaderBytes) st[lane] = lane == 0 ? (uint8_t)tid : (lane == 1 ? (uint8_t)n : 0);
+  if (lane_b < kHeaderBytes) st[lane_b] = lane_b == 0 ? (uint8_t)tid : (lane_b == 1 ? (uint8_t)n : 0);
   for (int k = 0; k < nk; ++k) {
     const int gi = gs + 4 * k;
-    if (t == 0 && gi < G) *reinterpret_cast<float*>(st + kHeaderBytes + 4 * gi) = scale_[k];
+    if (tk == 0 && gi < G) *reinterpret_cast<float*>(st + kHeaderBytes + 4 * gi) = scale_[k];
   }
   // LSB-first bit stream (bitpacking.py:14-27): bit j of item i = (token t,
   // group gi), i = t*G + gi, at bit i*b + j.  The theta section's dwords (hdr
   // = 8 + 4G is a multiple of 4) are cleared, then every item ORs its b bits
   // into the one or two dwords they fall in.
   uint32_t* thw = reinterpret_cast<uint32_t*>(st + hdr);
-  for (int w = lane; w < (tb + 3) / 4; w += kWave) thw[w] = 0u;
+  for (int w = lane_b; w < (tb + 3) / 4; w += kWave) thw[w] = 0u;
   wave_lds_sync();
   for (int k = 0; k < nk; ++k) {
     const int gi = gs + 4 * k;
     if (!tok_ok || gi >= G) continue;
     const uint32_t c = (uint32_t)best_[k];
-    const int o = (t * G + gi) * b, w = o >> 5, sh = o & 31;
+    const int o = (tk * G + gi) * b, w = o >> 5, sh = o & 31;
     __hip_atomic_fetch_or(thw + w, c << sh, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     if (sh + b > 32) __hip_atomic_fetch_or(thw + w + 1, c >> (32 - sh), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
@@ -589,14 +795,14 @@ __global__ __launch_bounds__(kEncWaves * 64) void encode_pages_kernel(EncodeArgs
   for (int k = 0; k < nk; ++k) {
     const int gi = gs + 4 * k;
     if (!tok_ok || gi >= G) continue;
-    const int item = t * G + gi;
+    const int item = tk * G + gi;
     const float safe = scale_[k] < 1e-8f ? 1e-8f : scale_[k];
     float qv = __fmul_rn(__fdiv_rn(rr_[k], safe), 127.0f);
     qv = __builtin_rintf(qv);
     qv = fminf(fmaxf(qv, -127.f), 127.f);
     st[hdr + tb + item] = (uint8_t)(int8_t)(int)qv;
-    if (a.r_out) a.r_out[((int64_t)p * kTile + t) * (DH / 16) + gi] = rr_[k];
-    if (a.code_out) a.code_out[((int64_t)p * kTile + t) * (DH / 16) + gi] = best_[k];
+    if (a.r_out) a.r_out[(pg * kTile + tk) * (DH / 16) + gi] = rr_[k];
+    if (a.code_out) a.code_out[(pg * kTile + tk) * (DH / 16) + gi] = best_[k];
   }
   wave_lds_sync();
   if (page_off >= 0 && page_off + size <= a.pages_bytes) {
@@ -604,8 +810,8 @@ __global__ __launch_bounds__(kEncWaves * 64) void encode_pages_kernel(EncodeArgs
     // (the next page may start right after it)
     const int nw = (page_off & 3) == 0 ? size >> 2 : 0;
     uint32_t* dw = reinterpret_cast<uint32_t*>(a.pages + page_off);
-    for (int i = lane; i < nw; i += kWave) dw[i] = reinterpret_cast<const uint32_t*>(st)[i];
-    for (int i = 4 * nw + lane; i < size; i += kWave) a.pages[page_off + i] = st[i];
+    for (int i = lane_b; i < nw; i += kWave) dw[i] = reinterpret_cast<const uint32_t*>(st)[i];
+    for (int i = 4 * nw + lane_b; i < size; i += kWave) a.pages[page_off + i] = st[i];
   }
 }
 
@@ -618,9 +824,13 @@ int launch_encode(const EncodeLaunch& L, hipStream_t stream) {
   a.pages = L.pages; a.pages_bytes = L.pages_bytes; a.v_pool = reinterpret_cast<__half*>(L.v_pool);
   a.num_vpages = L.num_vpages; a.r_out = L.r_out; a.code_out = L.code_out;
   a.order_n = L.order_n; a.codes_only = L.codes_only;
-  const dim3 grid((L.num_pages + kEncPages - 1) / kEncPages), block(kEncWaves * 64);
-  if (L.dh == 128) hipLaunchKernelGGL(encode_pages_kernel<128>, grid, block, 0, stream, a);
-  else hipLaunchKernelGGL(encode_pages_kernel<64>, grid, block, 0, stream, a);
+  const int per = L.dh == 128 ? enc_pages<128>() : enc_pages<64>();
+  const dim3 grid((L.num_pages + per - 1) / per), block(kEncWaves * 64);
+#define SPHKV_ENC(D, K, C) if (L.dh == D && (L.k_is_fp32 != 0) == K && (L.codes_only != 0) == C) \
+    hipLaunchKernelGGL((encode_pages_kernel<D, K, C>), grid, block, 0, stream, a);
+  SPHKV_ENC(128, false, false) SPHKV_ENC(128, true, false) SPHKV_ENC(128, false, true) SPHKV_ENC(128, true, true)
+  SPHKV_ENC(64, false, false) SPHKV_ENC(64, true, false) SPHKV_ENC(64, false, true) SPHKV_ENC(64, true, true)
+#undef SPHKV_ENC
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

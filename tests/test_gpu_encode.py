@@ -187,3 +187,48 @@ def test_encode_non_unit_codebooks_bit_exact(gpu, kind):
     assert (c[comp] == cpu["codes"][comp]).all(), f"{int((c[comp] != cpu['codes'][comp]).sum())} codes differ"
     assert (r[comp].view(np.uint32) == cpu["r"][comp].view(np.uint32)).all()
     assert (pool.pages.cpu().numpy() == cpu["pages"]).all()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("dh,H,L", [(128, 2, 203), (64, 3, 77)])
+def test_encode_small_gaps_scales_and_bit_patterns(gpu, dh, H, L, fp32):
+    # the MFMA ranking and its exact pass: gaps of 1e-7 to 1e-2 between the two
+    # best centroids (around the slack past which the ranking stands), ties of
+    # three centroids, groups from fp16 denormals to large, pages of every
+    # tier mixed in one workgroup, missing rows at the end of a workgroup; V and
+    # dense K of any bit pattern (negative zeros, infinities, NaNs) as they are
+    rng = np.random.default_rng(dh + fp32)
+    tier_of = [rng.choice(np.array([1, 2, 3, fmt.DENSE_TIER_ID], np.int32), size=L) for _ in range(H)]
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    K = np.zeros((H, L, dh), np.float32)
+    for h in range(H):
+        for t in range(L):
+            tid = int(tier_of[h][t])
+            if tid == fmt.DENSE_TIER_ID:
+                K[h, t] = rng.integers(0, 1 << 16, dh).astype(np.uint16).view(np.float16).astype(np.float32)
+                continue
+            cb = cbs[tid][h]
+            G, C, g = cb.shape
+            for j in range(G):
+                a, b, c = rng.choice(C, size=3, replace=False)
+                eps = np.float32(10.0 ** rng.uniform(-7, -2))
+                v = cb[j, a] + cb[j, b] * (1 - eps) + (cb[j, c] * (1 - eps) if t % 3 == 0 else 0)
+                K[h, t, j * g:(j + 1) * g] = v * np.float32(2.0 ** rng.integers(-22, 9))
+    dense = np.stack([t == fmt.DENSE_TIER_ID for t in tier_of])
+    if fp32:
+        K[dense] = np.where(np.isnan(K[dense]), 1.0, K[dense])       # (a NaN's payload is not kept by the conversion)
+    V = rng.integers(0, 1 << 16, (H, L, dh)).astype(np.uint16).view(np.float16)
+    plan = fmt.plan_pages(tier_of, None, 1, H, dh, 16, rng=rng)
+    wl = synth.Workload(name="gaps", dh=dh, num_kv=H, gqa=1, num_seqs=1, lengths=[L], rope_theta=5e5, codebooks=cbs,
+                        K=[K if fp32 else K.astype(np.float16)], V=[V], q=np.zeros((1, H, dh), np.float16),
+                        tier_of=tier_of, plan=plan)
+    log(f"encode gaps dh={dh} fp32={fp32} rows={plan.num_rows}")
+    pool, r_out, c_out = ops.build_pool_gpu(wl, gpu, with_codes=True)
+    torch.cuda.synchronize()
+    cpu = oracle.build_pool(wl, with_codes=True)
+    r, c = r_out.cpu().numpy(), c_out.cpu().numpy()
+    comp = plan.tier != fmt.DENSE_TIER_ID
+    assert (c[comp] == cpu["codes"][comp]).all(), f"{int((c[comp] != cpu['codes'][comp]).sum())} codes differ"
+    assert (r[comp].view(np.uint32) == cpu["r"][comp].view(np.uint32)).all()
+    assert (pool.pages.cpu().numpy() == cpu["pages"]).all()
+    assert (pool.v_pool.cpu().numpy().view(np.uint16) == cpu["v_pool"].view(np.uint16)).all()
