@@ -841,10 +841,9 @@ int sphkv_logits_lut(const float* q_lut, const uint8_t* theta_codes, const uint8
   return launch_status(sphkv::launch_lut_logits(L, (hipStream_t)stream), fn);
 }
 
-int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,
-                    const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
-                    int32_t max_blocks, float ema_beta, void* stream) {
-  const char* fn = "sphkv_omega_ema";
+static int omega_ema(const char* fn, const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,
+                     const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
+                     int32_t max_blocks, float ema_beta, void* ws, int64_t ws_bytes, void* stream) {
   if (num_kv < 0 || max_blocks < 0) return fail(SPHKV_EINVAL, "%s: negative size", fn);
   if (kv_groups < 1 || kv_groups > sphkv::kOmegaMaxGroups)
     return fail(SPHKV_EINVAL, "%s: kv_groups must be 1..%d", fn, sphkv::kOmegaMaxGroups);
@@ -852,8 +851,36 @@ int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_
   if (num_kv == 0 || max_blocks == 0) return ok();
   if (!m_q || !l_q || !omega_prev || !omega_out) return fail(SPHKV_EINVAL, "%s: null pointer argument", fn);
   sphkv::OmegaLaunch L{m_q, l_q, q_stride, page_stride, omega_prev, omega_out, num_kv, kv_groups, max_blocks,
-                       ema_beta};
+                       ema_beta, nullptr};
+  if (ws) {
+    const int64_t need = 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
+    if (ws_bytes < need || ((uintptr_t)ws & 7) != 0)
+      return fail(SPHKV_EINVAL, "%s: workspace needs %lld bytes, 8-byte aligned", fn, (long long)need);
+    if ((int64_t)num_kv * kv_groups * ((max_blocks + 255) / 256) < ((int64_t)1 << 31)) L.ws = static_cast<float*>(ws);
+  }
   return launch_status(sphkv::launch_omega(L, (hipStream_t)stream), fn);
+}
+
+int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,
+                    const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
+                    int32_t max_blocks, float ema_beta, void* stream) {
+  return omega_ema("sphkv_omega_ema", m_q, l_q, q_stride, page_stride, omega_prev, omega_out, num_kv, kv_groups,
+                   max_blocks, ema_beta, nullptr, 0, stream);
+}
+
+int64_t sphkv_omega_ema_workspace_bytes(int32_t num_kv, int32_t kv_groups, int32_t max_blocks) {
+  if (num_kv < 0 || max_blocks < 0 || kv_groups < 1 || kv_groups > sphkv::kOmegaMaxGroups) return -1;
+  // one workgroup per kv head reads up to kOmegaSplitBlocks pages as fast as
+  // two kernels do
+  if (max_blocks <= sphkv::kOmegaSplitBlocks) return 0;
+  return 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
+}
+
+int sphkv_omega_ema_ws(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,
+                       const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
+                       int32_t max_blocks, float ema_beta, void* workspace, int64_t workspace_bytes, void* stream) {
+  return omega_ema("sphkv_omega_ema_ws", m_q, l_q, q_stride, page_stride, omega_prev, omega_out, num_kv, kv_groups,
+                   max_blocks, ema_beta, workspace, workspace_bytes, stream);
 }
 
 int sphkv_build_layer_pool(const float* r, const int32_t* theta, int64_t n_elems, const uint16_t* v,

@@ -117,7 +117,14 @@ struct OmegaLaunch {
   const float* m; const float* l; int64_t q_stride, page_stride;   // element strides of the (m, l) views
   const float* omega_prev; float* omega_out;                        // [num_kv, max_blocks]; may alias
   int32_t num_kv, kv_groups, max_blocks; float beta;
+  float* ws;                                                        // omega_workspace_floats() floats, or NULL: one kernel
 };
+constexpr int kOmegaChunk = 256;         // pages per workgroup of the two-kernel form
+constexpr int kOmegaSplitBlocks = 512;   // most pages of the one-kernel form when a workspace is offered
+// (max, sum) of each (q head, chunk), then (m, l) of each (q head, page)
+inline int64_t omega_workspace_floats(int32_t num_kv, int32_t kv_groups, int32_t max_blocks) {
+  return 2 * (int64_t)num_kv * kv_groups * ((max_blocks + kOmegaChunk - 1) / kOmegaChunk + (int64_t)max_blocks);
+}
 
 constexpr int kPoolBuildMaxG = 256;
 struct PoolBuildLaunch {

@@ -1244,10 +1244,84 @@ __global__ __launch_bounds__(1024) void omega_ema_fast_kernel(OmegaLaunch a, int
   }
 }
 
+// Two-kernel form.  The (m, l) pairs lie a whole partial apart (520 bytes at dh
+// 128), so every pair is a line of its own and a workgroup that reads a kv
+// head's 2,048 pages x 4 q heads is bound by its CU's line rate (22.9 us).
+// Here a workgroup reads 256 pages of one q head, leaves their maximum and sum
+// and a packed copy of the pairs; the second kernel folds the chunks' pairs
+// and blends 256 pages of a kv head.  Same formula; the sums relative to a
+// chunk's maximum are rescaled to the head's.
+__global__ __launch_bounds__(kOmegaChunk) void omega_chunk_kernel(OmegaLaunch a, int nch, int adjacent) {
+  __shared__ float red[kOmegaChunk / 64];
+  const int hq = blockIdx.x / nch, c = blockIdx.x - hq * nch;
+  const int p = c * kOmegaChunk + threadIdx.x;
+  const bool ok = p < a.max_blocks;
+  const int64_t o = (int64_t)hq * a.q_stride + (int64_t)(ok ? p : 0) * a.page_stride;
+  float m, l;
+  if (adjacent) {
+    const float2 v = *reinterpret_cast<const float2*>(a.m + o);
+    m = v.x; l = v.y;
+  } else {
+    m = a.m[o]; l = a.l[o];
+  }
+  l = ok ? l : 0.f;
+  m = (ok && l > 0.f) ? m : -1e30f;                    // invalid pages do not win the max
+  float2* part = reinterpret_cast<float2*>(a.ws);
+  float2* pairs = part + (int64_t)a.num_kv * a.kv_groups * nch;
+  if (ok) pairs[(int64_t)hq * a.max_blocks + p] = float2{m, l};
+  const float mx = block_reduce(m, true, red);
+  const float z = block_reduce(expf(fmaxf(m - mx, -60.f)) * l, false, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = float2{mx, z};
+}
+
+__global__ __launch_bounds__(kOmegaChunk) void omega_blend_kernel(OmegaLaunch a, int nch) {
+  __shared__ float mx_s[kOmegaMaxGroups], z_s[kOmegaMaxGroups];
+  const int h = blockIdx.x / nch, c = blockIdx.x - h * nch;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float2* part = reinterpret_cast<const float2*>(a.ws);
+  const float2* pairs = part + (int64_t)a.num_kv * a.kv_groups * nch;
+  for (int r = wave; r < a.kv_groups; r += kOmegaChunk / 64) {
+    const float2* pr = part + ((int64_t)h * a.kv_groups + r) * nch;
+    float mx = -1e30f, z = 0.f;
+    for (int k = lane; k < nch; k += 64) {
+      const float2 v = pr[k];
+      const float mn = fmaxf(mx, v.x);
+      z = z * expf(fmaxf(mx - mn, -80.f)) + v.y * expf(fmaxf(v.x - mn, -80.f));
+      mx = mn;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const float mo = __shfl_xor(mx, o, 64), zo = __shfl_xor(z, o, 64);
+      const float mn = fmaxf(mx, mo);
+      z = z * expf(fmaxf(mx - mn, -80.f)) + zo * expf(fmaxf(mo - mn, -80.f));
+      mx = mn;
+    }
+    if (lane == 0) { mx_s[r] = mx; z_s[r] = fmaxf(z, 1e-12f); }
+  }
+  __syncthreads();
+  const int p = c * kOmegaChunk + threadIdx.x;
+  if (p >= a.max_blocks) return;
+  float s = 0.f;
+  for (int r = 0; r < a.kv_groups; ++r) {
+    const float2 v = pairs[((int64_t)h * a.kv_groups + r) * a.max_blocks + p];
+    s += expf(fmaxf(v.x - mx_s[r], -60.f)) * v.y / z_s[r];
+  }
+  const float mass = s / (float)a.kv_groups;
+  const int64_t o = (int64_t)h * a.max_blocks + p;
+  a.omega_out[o] = a.omega_prev[o] * a.beta + mass * (1.f - a.beta);
+}
+
 int launch_omega(const OmegaLaunch& L, hipStream_t stream) {
   if (L.num_kv <= 0 || L.max_blocks <= 0) return 0;
   // (an 8-byte (m, l) load needs l right after m and 8-byte alignment at every page)
   const bool adjacent = L.l == L.m + 1 && ((uintptr_t)L.m % 8) == 0 && L.q_stride % 2 == 0 && L.page_stride % 2 == 0;
+  if (L.ws) {
+    const int nch = (L.max_blocks + kOmegaChunk - 1) / kOmegaChunk;
+    hipLaunchKernelGGL(omega_chunk_kernel, dim3(L.num_kv * L.kv_groups * nch), dim3(kOmegaChunk), 0, stream, L, nch,
+                       (int)adjacent);
+    hipLaunchKernelGGL(omega_blend_kernel, dim3(L.num_kv * nch), dim3(kOmegaChunk), 0, stream, L, nch);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+  }
   if (L.kv_groups <= 4 && L.max_blocks <= 4096) {
     if (L.max_blocks <= 2048)
       hipLaunchKernelGGL((omega_ema_fast_kernel<2, 4>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);

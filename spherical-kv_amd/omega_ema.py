@@ -6,7 +6,7 @@ Same argument meaning as the reference: m_q, l_q are the [num_q, max_blocks]
 (m, l) views of the decode's partial_scratch ([..., 0] and [..., 1]); the
 strided views are read in place.  Returns the new omega [num_kv, max_blocks]
 fp32 (out of place, like the reference; pass `out=omega_prev` to update in
-place).  One HIP kernel; raises if libsphkv.so is missing.
+place).  One HIP kernel (two past 512 blocks); raises if libsphkv.so is missing.
 """
 from __future__ import annotations
 
@@ -43,9 +43,14 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
         out = torch.empty_like(omega_prev)
     elif out.dtype != torch.float32 or not out.is_contiguous() or out.shape != omega_prev.shape:
         raise ValueError("out must be a contiguous fp32 tensor shaped like omega_prev")
-    rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(),
-                              out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),
-                              sphkv_lib.current_stream())
+    args = (m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(), out.data_ptr(),
+            int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta))
+    if args[8] > 512:                                    # long tables: two kernels over scratch of this call's stream
+        nws = _lib.sphkv_omega_ema_workspace_bytes(*args[6:9])
+        ws = torch.empty(max(nws, 8), dtype=torch.uint8, device=out.device)
+        rc = _lib.sphkv_omega_ema_ws(*args, ws.data_ptr(), max(nws, 8), sphkv_lib.current_stream())
+    else:
+        rc = _lib.sphkv_omega_ema(*args, sphkv_lib.current_stream())
     check(rc, "omega_ema")
     return out
 

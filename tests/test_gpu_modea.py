@@ -229,3 +229,29 @@ def test_omega_ema_kernel_forms(gpu, num_kv, kv_groups, max_blocks, adjacent):
     got = omega_ema.omega_ema(mt, lt, _t(prev, gpu), num_kv, kv_groups, max_blocks, 0.9).cpu().numpy()
     want = oracle.omega_ema(m, l, prev, num_kv, kv_groups, 0.9)
     np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("num_kv,kv_groups,max_blocks", [(2, 4, 512), (2, 4, 513), (1, 9, 768), (3, 1, 1025), (1, 2, 20000)])
+def test_omega_ema_one_and_two_kernels(gpu, num_kv, kv_groups, max_blocks):
+    # the form with a workspace (chunks of 256 pages: a whole last one, one
+    # page more, more chunks than lanes) and the one without agree with the
+    # oracle; a whole chunk and a whole head without valid pages; in place
+    import omega_ema
+    import sphkv_lib
+    rng = np.random.default_rng(max_blocks)
+    nq = num_kv * kv_groups
+    m = (rng.standard_normal((nq, max_blocks)) * 20).astype(np.float32)
+    l = np.where(rng.random((nq, max_blocks)) < 0.8, rng.random((nq, max_blocks)) * 3, 0.0).astype(np.float32)
+    l[:, 256:512] = 0.0
+    l[-1] = 0.0
+    prev = rng.random((num_kv, max_blocks)).astype(np.float32)
+    ml = torch.from_numpy(np.stack([m, l], axis=-1)).to(gpu)
+    want = oracle.omega_ema(m, l, prev, num_kv, kv_groups, 0.9)
+    out = _t(prev, gpu)
+    omega_ema.omega_ema(ml[..., 0], ml[..., 1], out, num_kv, kv_groups, max_blocks, 0.9, out=out)
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=1e-5, atol=1e-7)
+    one = _t(prev, gpu)
+    rc = sphkv_lib.load().sphkv_omega_ema(ml.data_ptr(), ml.data_ptr() + 4, ml.stride(0), 2, one.data_ptr(),
+                                          one.data_ptr(), num_kv, kv_groups, max_blocks, 0.9, sphkv_lib.current_stream())
+    assert rc == 0
+    np.testing.assert_allclose(one.cpu().numpy(), want, rtol=1e-5, atol=1e-7)
