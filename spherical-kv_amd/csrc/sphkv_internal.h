@@ -140,7 +140,7 @@ struct PlanLaunch {
   const uint8_t* tier_of; int64_t tier_stride;   // [num_sh, >= L_s] tier id per token
   const int32_t* lens;                           // [num_seqs] tokens per sequence
   int32_t max_len;                               // >= every lens[s]: sizes the token chunks
-  int32_t nchunks;                               // set by launch_plan
+  int32_t chunk, nchunks;                        // set by launch_plan
   const int32_t* pos; int64_t pos_stride;        // [num_seqs, >= L_s] positions, or null (token index)
   const int64_t* row_base;                       // [num_sh] K row of token 0, or null (no src_rows)
   int32_t num_sh, num_kv, dh;

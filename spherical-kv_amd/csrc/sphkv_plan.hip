@@ -17,12 +17,14 @@
 // (config.py:14-15); a caller whose recents carry another tier than its
 // sinks gets index order.
 //
-// Kernels (a (sequence, head)'s tokens are cut into chunks of kPlanChunk):
+// Kernels (a (sequence, head)'s tokens are cut into chunks, plan_chunk).  All
+// three are bound by the round trips of a chain of small loads, so the tiers of
+// a chunk's tokens are loaded together, before anything depends on them:
 //   plan_count_kernel  per (sequence, head, chunk): tokens and first index
 //                      per tier, by wave ballots
-//   plan_scan_kernel   one workgroup: per (sequence, head) a wave scans its
-//                      chunks' counts into rank bases (64 chunks per load) and
-//                      sets the tier order and rows; then the tier runs are
+//   plan_scan_kernel   one workgroup: per (sequence, head) a group of lanes
+//                      scans its chunks' counts into rank bases and sets the
+//                      tier order and rows; then the tier runs are
 //                      placed back to back by a block-wide scan of placement
 //                      maps (below), each thread taking a contiguous span of
 //                      (sequence, head) ranges
@@ -72,7 +74,14 @@ __device__ __forceinline__ int64_t place(int64_t off, int k) {
 enum : int { kCnt = 0, kFirst = 4, kRows = 8, kOrder = 9, kRunStart = 10, kRowStart = 14, kRec = 16 };
 // per chunk: counts (then rank bases), first index, invalid ids, sequence-length flag
 enum : int { kChCnt = 0, kChFirst = 4, kChBad = 8, kChLen = 9, kChRec = 12 };
-constexpr int kPlanChunk = 2048;
+// Tokens per chunk (a workgroup of the count and fill kernels): 2,048, or 512
+// where the longer ones would leave CUs without a workgroup.
+constexpr int kPlanChunk = 2048, kPlanChunkShort = 512, kPlanFewChunks = 256;
+constexpr int kPlanIters = kPlanChunk / kPlanThreads;
+inline int plan_chunk(int num_sh, int max_len) {
+  const int64_t n = max_len <= 0 ? 1 : ((int64_t)max_len + kPlanChunk - 1) / kPlanChunk;
+  return (int64_t)num_sh * n <= kPlanFewChunks ? kPlanChunkShort : kPlanChunk;
+}
 constexpr int kScanThreads = 1024;
 constexpr int64_t kMaxOff = 0x7FFFFF00LL;   // byte offsets stay int32
 
@@ -94,22 +103,20 @@ __device__ __forceinline__ Place run_map(int k, int n, int dh) {
   return k == 3 ? Place{run_bytes(k, n, dh) - kHeader, kHeader, 0} : Place{run_bytes(k, n, dh), 0, 0};
 }
 
-__device__ __forceinline__ int wave_scan_incl(int v, int lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
+// Inclusive scan, minimum and sum over aligned groups of `width` lanes (a power of two).
+__device__ __forceinline__ int group_scan_incl(int v, int lane, int width) {
+  for (int d = 1; d < width; d <<= 1) {
     const int t = __shfl_up(v, d, 64);
-    if (lane >= d) v += t;
+    if ((lane & (width - 1)) >= d) v += t;
   }
   return v;
 }
-__device__ __forceinline__ int wave_min(int v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
+__device__ __forceinline__ int group_min(int v, int width) {
+  for (int d = width >> 1; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
   return v;
 }
-__device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+__device__ __forceinline__ int group_sum(int v, int width) {
+  for (int d = width >> 1; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
   return v;
 }
 
@@ -118,18 +125,39 @@ __device__ __forceinline__ int32_t* ch_rec(const PlanLaunch& a, int sh, int c) {
   return a.work + (int64_t)a.num_sh * kRec + ((int64_t)sh * a.nchunks + c) * kChRec;
 }
 
+// Tier slots of the thread's tokens t0 + threadIdx.x + 256 i < t1 of a chunk
+// (-1 past it), their bytes all in flight together.
+__device__ __forceinline__ void load_tiers(const PlanLaunch& a, int sh, int t0, int t1, int (&k)[kPlanIters]) {
+  const uint8_t* t_of = a.tier_of + (int64_t)sh * a.tier_stride;
+  int raw[kPlanIters];
+  if (t0 >= a.max_len) {                                 // max_len 0: the rows are empty
+    for (int it = 0; it < kPlanIters; ++it) k[it] = -1;
+    return;
+  }
+#pragma unroll
+  for (int it = 0; it < kPlanIters; ++it) {
+    const int t = t0 + it * kPlanThreads + (int)threadIdx.x;
+    raw[it] = t_of[t < t1 ? t : t0];                     // t0 < max_len, the row's width
+  }
+#pragma unroll
+  for (int it = 0; it < kPlanIters; ++it) k[it] = t0 + it * kPlanThreads + (int)threadIdx.x < t1 ? tier_slot(raw[it]) : -1;
+}
+
 }  // namespace
 
 __global__ __launch_bounds__(kPlanThreads) void plan_count_kernel(PlanLaunch a) {
   __shared__ int wc[kPlanThreads / 64][4], wf[kPlanThreads / 64][4], wbad[kPlanThreads / 64];
   const int sh = blockIdx.x / a.nchunks, c = blockIdx.x % a.nchunks, s = sh / a.num_kv;
-  const int L = min(a.lens[s], a.max_len), t0 = c * kPlanChunk, t1 = min(L, t0 + kPlanChunk);
-  const uint8_t* t_of = a.tier_of + (int64_t)sh * a.tier_stride;
+  const int L = min(a.lens[s], a.max_len), t0 = c * a.chunk, t1 = min(L, t0 + a.chunk);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int k_of[kPlanIters];
+  load_tiers(a, sh, t0, t1, k_of);
   int cnt[4] = {0, 0, 0, 0}, first[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, bad = 0;
-  for (int b = t0; b < t1; b += kPlanThreads) {        // wave-uniform trip count
-    const int t = b + threadIdx.x;
-    const int k = t < t1 ? tier_slot(t_of[t]) : -1;
+#pragma unroll
+  for (int it = 0; it < kPlanIters; ++it) {
+    const int b = t0 + it * kPlanThreads;
+    if (b >= t1) break;                                  // workgroup-uniform
+    const int k = k_of[it];
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
       const uint64_t m = __builtin_amdgcn_ballot_w64(k == kk);
@@ -183,43 +211,49 @@ __global__ __launch_bounds__(kScanThreads) void plan_scan_kernel(PlanLaunch a) {
   const bool cached = a.num_sh <= kScanThreads;
   if (t == 0) { nbad = 0; nflag = 0; }
   __syncthreads();
-  // (1) a wave per (sequence, head): its chunks' exclusive rank bases per
-  // tier, 64 chunks per step, then totals, first indices, tier order, rows
-  for (int sh = wave; sh < a.num_sh; sh += kScanThreads / 64) {
+  // (1) per (sequence, head) a group of lanes, one chunk each (a whole wave and
+  // 64 chunks per step where there are more): the chunks' exclusive rank
+  // bases per tier, then totals, first indices, tier order, rows.  A wave per
+  // (sequence, head) took 16 of them at a time, each a round trip: 43.5 us at
+  // 128 of 6 chunks.
+  int width = 1;
+  while (width < a.nchunks && width < 64) width <<= 1;
+  const int gpw = 64 / width, gl = lane & (width - 1);   // groups per wave, lane in its group
+  for (int sb = wave * gpw; sb < a.num_sh; sb += (kScanThreads / 64) * gpw) {   // wave-uniform trip count
+    const int sh = sb + lane / width;
+    const bool sh_ok = sh < a.num_sh;
     int carry[4] = {0, 0, 0, 0}, first[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF}, bad = 0, flag = 0;
-    for (int c0 = 0; c0 < a.nchunks; c0 += 64) {          // wave-uniform trip count
-      const int c = c0 + lane;
-      int32_t* r = c < a.nchunks ? ch_rec(a, sh, c) : nullptr;
+    for (int c0 = 0; c0 < a.nchunks; c0 += width) {       // wave-uniform trip count
+      const int c = c0 + gl;
+      int32_t* r = sh_ok && c < a.nchunks ? ch_rec(a, sh, c) : nullptr;
       int n[4], f[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) { n[k] = r ? r[kChCnt + k] : 0; f[k] = r ? r[kChFirst + k] : 0x7FFFFFFF; }
       if (r) { bad += r[kChBad]; flag |= r[kChLen]; }
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int incl = wave_scan_incl(n[k], lane);
+        const int incl = group_scan_incl(n[k], lane, width);
         if (r) r[kChCnt + k] = carry[k] + incl - n[k];
-        carry[k] += __shfl(incl, 63, 64);
+        carry[k] += __shfl(incl, lane | (width - 1), 64);
         first[k] = min(first[k], f[k]);
       }
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) first[k] = wave_min(first[k]);
-    bad = wave_sum(bad);
-    flag = wave_sum(flag);
-    if (lane == 0) {
-      int order = 0, n_runs = 0, rows = 0;
-      bool used[4] = {false, false, false, false};
-      for (int q = 0; q < 4; ++q) {                      // tiers by first appearance
-        int best = -1;
-        for (int k = 0; k < 4; ++k)
-          if (!used[k] && carry[k] > 0 && (best < 0 || first[k] < first[best])) best = k;
-        if (best < 0) break;
-        used[best] = true;
-        order |= best << (4 * n_runs);
-        ++n_runs;
-        rows += (carry[best] + 15) / 16;
+    for (int k = 0; k < 4; ++k) first[k] = group_min(first[k], width);
+    bad = group_sum(bad, width);
+    flag = group_sum(flag, width);
+    if (gl == 0 && sh_ok) {
+      // tiers by first appearance: the place of each among the used ones
+      int order = 0xFFFF, rows = 0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        if (carry[k] <= 0) continue;
+        int q = 0;
+#pragma unroll
+        for (int o = 0; o < 4; ++o) q += o != k && carry[o] > 0 && (first[o] < first[k] || (first[o] == first[k] && o < k));
+        order = (order & ~(0xF << (4 * q))) | (k << (4 * q));
+        rows += (carry[k] + 15) / 16;
       }
-      for (int q = n_runs; q < 4; ++q) order |= 0xF << (4 * q);
       int32_t* rec = sh_rec(a, sh);
       for (int k = 0; k < 4; ++k) { rec[kCnt + k] = carry[k]; rec[kFirst + k] = first[k]; }
       rec[kRows] = rows;
@@ -307,25 +341,53 @@ __global__ __launch_bounds__(kScanThreads) void plan_scan_kernel(PlanLaunch a) {
 }
 
 __global__ __launch_bounds__(kPlanThreads) void plan_fill_kernel(PlanLaunch a) {
-  __shared__ int page0[4], npages[4], run_start[4], base[4], wsum[kPlanThreads / 64][4];
+  constexpr int NW = kPlanThreads / 64;
+  __shared__ int page0[4], npages[4], run_start[4], srec[kRec], scnt[4], wsum[4][kPlanIters * NW];
   const int sh = blockIdx.x / a.nchunks, c = blockIdx.x % a.nchunks, s = sh / a.num_kv;
-  const int32_t* rec = sh_rec(a, sh);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // the records and every token's tier share one round trip
+  const int L = min(a.lens[s], a.max_len), t0 = c * a.chunk, t1 = min(L, t0 + a.chunk);
+  const int64_t rb = a.row_base ? a.row_base[sh] : 0;
+  int k_of[kPlanIters];
+  load_tiers(a, sh, t0, t1, k_of);
+  if (threadIdx.x < kRec) srec[threadIdx.x] = sh_rec(a, sh)[threadIdx.x];
+  else if (threadIdx.x < kRec + 4) scnt[threadIdx.x - kRec] = ch_rec(a, sh, c)[kChCnt + threadIdx.x - kRec];
+  // tokens of each tier per (256-token step, wave); a token's rank among its wave's
+  int below[kPlanIters];
+#pragma unroll
+  for (int it = 0; it < kPlanIters; ++it) {
+    below[it] = 0;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(k_of[it] == kk);
+      if (lane == 0) wsum[kk][it * NW + wave] = __builtin_popcountll(m);
+      if (k_of[it] == kk) below[it] = __builtin_popcountll(m & ((1ull << lane) - 1ull));
+    }
+  }
+  __syncthreads();
+  const int32_t* rec = srec;
   const int row0 = rec[kRowStart];
   const int rows = rec[kRows];
   if (row0 < 0 || row0 + rows > a.max_rows) return;       // outputs too small: nothing is written
-  if (threadIdx.x == 0) {
-    int p = 0;
-    for (int k = 0; k < 4; ++k) { page0[k] = -1; npages[k] = 0; }
-    for (int q = 0; q < 4; ++q) {
-      const int k = (rec[kOrder] >> (4 * q)) & 0xF;
-      if (k == 0xF) break;
-      page0[k] = p;
-      npages[k] = (rec[kCnt + k] + 15) / 16;
-      run_start[k] = rec[kRunStart + q];
-      p += npages[k];
+  {
+    // wave kk: tier kk's counts into rank bases (exclusive, after the earlier
+    // chunks'); its first page and run start
+    static_assert(NW == 4 && kPlanIters * NW <= 64, "one wave per tier, one lane per step and wave");
+    const int v = lane < kPlanIters * NW ? wsum[wave][lane] : 0;
+    const int incl = group_scan_incl(v, lane, 64);
+    if (lane < kPlanIters * NW) wsum[wave][lane] = scnt[wave] + incl - v;
+    if (lane == 0) {
+      int p = 0, first_page = -1, run = 0;
+      for (int q = 0; q < 4; ++q) {
+        const int k = (rec[kOrder] >> (4 * q)) & 0xF;
+        if (k == 0xF) break;
+        if (k == wave) { first_page = p; run = rec[kRunStart + q]; }
+        p += (rec[kCnt + k] + 15) / 16;
+      }
+      page0[wave] = first_page;
+      npages[wave] = first_page < 0 ? 0 : (rec[kCnt + wave] + 15) / 16;
+      run_start[wave] = run;
     }
-    const int32_t* cr = ch_rec(a, sh, c);
-    for (int k = 0; k < 4; ++k) base[k] = cr[kChCnt + k];
   }
   __syncthreads();
   // this chunk's share of the page rows: tier, count, pointer-table row,
@@ -362,45 +424,29 @@ __global__ __launch_bounds__(kPlanThreads) void plan_fill_kernel(PlanLaunch a) {
     }
   }
   // each kept token of the chunk: rank within its tier -> (page, slot)
-  const int L = min(a.lens[s], a.max_len), t0 = c * kPlanChunk, t1 = min(L, t0 + kPlanChunk);
-  const uint8_t* t_of = a.tier_of + (int64_t)sh * a.tier_stride;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t rb = a.row_base ? a.row_base[sh] : 0;
-  for (int b0 = t0; b0 < t1; b0 += kPlanThreads) {
-    const int t = b0 + threadIdx.x;
-    const int k = t < t1 ? tier_slot(t_of[t]) : -1;
-    int below = 0;
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const uint64_t m = __builtin_amdgcn_ballot_w64(k == kk);
-      if (lane == 0) wsum[wave][kk] = __builtin_popcountll(m);
-      if (k == kk) below = __builtin_popcountll(m & ((1ull << lane) - 1ull));
-    }
-    __syncthreads();
-    if (k >= 0) {
-      int r = base[k] + below;
-      for (int w = 0; w < wave; ++w) r += wsum[w][k];
-      const int row = row0 + page0[k] + r / 16, q = r % 16;
-      a.tokens[(int64_t)row * 16 + q] = t;
-      a.positions[(int64_t)row * 16 + q] = a.pos ? a.pos[(int64_t)s * a.pos_stride + t] : t;
-      if (a.src_rows) a.src_rows[(int64_t)row * 16 + q] = rb + t;
-    }
-    __syncthreads();
-    if (threadIdx.x < 4)
-      for (int w = 0; w < kPlanThreads / 64; ++w) base[threadIdx.x] += wsum[w][threadIdx.x];
-    __syncthreads();
+  for (int it = 0; it < kPlanIters; ++it) {
+    const int t = t0 + it * kPlanThreads + (int)threadIdx.x, k = k_of[it];
+    if (k < 0) continue;
+    const int r = wsum[k][it * NW + wave] + below[it];
+    const int64_t o = (int64_t)(row0 + page0[k] + r / 16) * 16 + r % 16;
+    a.tokens[o] = t;
+    a.positions[o] = a.pos ? a.pos[(int64_t)s * a.pos_stride + t] : t;
+    if (a.src_rows) a.src_rows[o] = rb + t;
   }
 }
 
 int64_t plan_work_ints(int num_sh, int max_len) {
-  const int64_t nch = max_len <= 0 ? 1 : (max_len + kPlanChunk - 1) / kPlanChunk;
+  const int chunk = plan_chunk(num_sh, max_len);
+  const int64_t nch = max_len <= 0 ? 1 : ((int64_t)max_len + chunk - 1) / chunk;
   return (int64_t)num_sh * kRec + (int64_t)num_sh * nch * kChRec;
 }
 
 int launch_plan(const PlanLaunch& L0, int phase, hipStream_t stream) {
   if (L0.num_sh <= 0) return 0;
   PlanLaunch L = L0;
-  L.nchunks = L.max_len <= 0 ? 1 : (L.max_len + kPlanChunk - 1) / kPlanChunk;
+  L.chunk = plan_chunk(L.num_sh, L.max_len);
+  L.nchunks = L.max_len <= 0 ? 1 : (int)(((int64_t)L.max_len + L.chunk - 1) / L.chunk);
   const int64_t grid = (int64_t)L.num_sh * L.nchunks;
   if (grid > 0x7FFFFFFF) return -1;
   if (phase == 0) {

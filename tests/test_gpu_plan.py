@@ -175,3 +175,18 @@ def test_device_plan_follows_allocate_order_at_reference_defaults(gpu):
     dp = ops.plan_pages_gpu(t, lens, num_kv, dh, row_base=torch.from_numpy(base).to(gpu))
     log(f"sink 4 / recent 256: rows {dp.rows} pool bytes {dp.pages_bytes}")
     _check(dp, tier_of, lengths, num_kv, base, sink=4, recent=256)
+
+
+@pytest.mark.parametrize("lengths,num_kv", [
+    ([512], 8), ([513], 8), ([1], 1), ([33000], 1),            # chunks of 512: one, two, none whole, 65
+    ([3, 0, 1500], 4),                                         # lane groups of 4, two chunks unused
+    ([1200] * 33, 8), ([2049, 1, 4097] * 43, 2)])              # chunks of 2,048: 1 and 3 per range, ranges without tokens in some
+def test_device_plan_chunk_lengths(gpu, lengths, num_kv):
+    rng = np.random.default_rng(len(lengths) + lengths[0])
+    ids = np.array([0, 1, 2, 3, fmt.DENSE_TIER_ID])
+    tier_of = [rng.choice(ids, size=L, p=[0.1, 0.4, 0.3, 0.1, 0.1]).astype(np.int32) for L in lengths for _ in range(num_kv)]
+    t, lens, _ = _device_inputs(tier_of, lengths, num_kv, gpu)
+    base = _row_base(lengths, num_kv)
+    dp = ops.plan_pages_gpu(t, lens, num_kv, 64, row_base=torch.from_numpy(base).to(gpu))
+    log(f"chunk lengths: {len(tier_of)} ranges of up to {max(lengths)}: rows {dp.rows}")
+    _check(dp, tier_of, lengths, num_kv, base)
