@@ -31,6 +31,8 @@
 //                      out = acc / (l + 1e-8).
 //   qlut_kernel        the per-query LUT [num_q, num_tiers, G_max, cb_max].
 //   lut_logits_kernel  logits from a given LUT (new_fused_decode.py:22-43).
+#include <type_traits>
+
 #include "sphkv_common.h"
 #include "sphkv_internal.h"
 
@@ -1165,15 +1167,18 @@ __global__ __launch_bounds__(256) void omega_ema_kernel(OmegaLaunch a) {
   }
 }
 
-// Single-pass form for kv_groups <= KG (4 or 8) and max_blocks <= 1024 * PPT:
-// 1024 threads per kv head, each holding the (m, l) of its PPT pages for every
+// Single-pass form for kv_groups <= KG (4 or 8) and max_blocks <= NT * PPT: NT
+// threads per kv head, each holding the (m, l) of its PPT pages for every
 // q head of the group in registers (read once; one 8-byte load per pair when
 // l directly follows m, as in partial_scratch; no load for q heads past
 // kv_groups), the group's maxima and sums reduced together.  Same formula as
-// omega_ema_kernel.
-template <int PPT, int KG>
-__global__ __launch_bounds__(1024) void omega_ema_fast_kernel(OmegaLaunch a, int adjacent) {
-  __shared__ float red[16][KG];
+// omega_ema_kernel.  Up to 256 blocks NT is 256: the chain of barriers and
+// shuffles is what such a call costs, and 4 waves pass it sooner than 16 (16
+// kv heads, 64 blocks: 7.0 -> 4.0 us).
+template <int PPT, int KG, int NT>
+__global__ __launch_bounds__(NT) void omega_ema_fast_kernel(OmegaLaunch a, int adjacent) {
+  constexpr int NW = NT / 64;
+  __shared__ float red[NW][KG];
   const int h = blockIdx.x, kg = a.kv_groups;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   float mv[KG][PPT], lv[KG][PPT];
@@ -1181,7 +1186,7 @@ __global__ __launch_bounds__(1024) void omega_ema_fast_kernel(OmegaLaunch a, int
   for (int r = 0; r < KG; ++r) {
 #pragma unroll
     for (int i = 0; i < PPT; ++i) {
-      const int p = threadIdx.x + 1024 * i;
+      const int p = threadIdx.x + NT * i;
       const bool ok = r < kg && p < a.max_blocks;
       const int64_t o = (int64_t)(h * kg + (r < kg ? r : 0)) * a.q_stride + (int64_t)(ok ? p : 0) * a.page_stride;
       float m = 0.f, l = 0.f;
@@ -1211,7 +1216,7 @@ __global__ __launch_bounds__(1024) void omega_ema_fast_kernel(OmegaLaunch a, int
 #pragma unroll
     for (int r = 0; r < KG; ++r) {
       float t = red[0][r];
-      for (int w = 1; w < 16; ++w) t = is_max ? fmaxf(t, red[w][r]) : t + red[w][r];
+      for (int w = 1; w < NW; ++w) t = is_max ? fmaxf(t, red[w][r]) : t + red[w][r];
       v[r] = t;
     }
   };
@@ -1232,7 +1237,7 @@ __global__ __launch_bounds__(1024) void omega_ema_fast_kernel(OmegaLaunch a, int
   reduce(z, false);
 #pragma unroll
   for (int i = 0; i < PPT; ++i) {
-    const int p = threadIdx.x + 1024 * i;
+    const int p = threadIdx.x + NT * i;
     if (p >= a.max_blocks) continue;
     float s = 0.f;
 #pragma unroll
@@ -1322,16 +1327,18 @@ int launch_omega(const OmegaLaunch& L, hipStream_t stream) {
     hipLaunchKernelGGL(omega_blend_kernel, dim3(L.num_kv * nch), dim3(kOmegaChunk), 0, stream, L, nch);
     return hipGetLastError() == hipSuccess ? 0 : -1;
   }
-  if (L.kv_groups <= 4 && L.max_blocks <= 4096) {
-    if (L.max_blocks <= 2048)
-      hipLaunchKernelGGL((omega_ema_fast_kernel<2, 4>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
+  auto fast = [&](auto kg) {
+    constexpr int KG = decltype(kg)::value;
+    if (L.max_blocks <= 256)
+      hipLaunchKernelGGL((omega_ema_fast_kernel<1, KG, 256>), dim3(L.num_kv), dim3(256), 0, stream, L, (int)adjacent);
+    else if (L.max_blocks <= 2048)
+      hipLaunchKernelGGL((omega_ema_fast_kernel<2, KG, 1024>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
     else
-      hipLaunchKernelGGL((omega_ema_fast_kernel<4, 4>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
-  } else if (L.kv_groups <= 8 && L.max_blocks <= 4096) {
-    if (L.max_blocks <= 2048)
-      hipLaunchKernelGGL((omega_ema_fast_kernel<2, 8>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
-    else
-      hipLaunchKernelGGL((omega_ema_fast_kernel<4, 8>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
+      hipLaunchKernelGGL((omega_ema_fast_kernel<4, KG, 1024>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
+  };
+  if (L.kv_groups <= 8 && L.max_blocks <= 4096) {
+    if (L.kv_groups <= 4) fast(std::integral_constant<int, 4>());
+    else fast(std::integral_constant<int, 8>());
   } else {
     hipLaunchKernelGGL(omega_ema_kernel, dim3(L.num_kv), dim3(256), 0, stream, L);
   }

@@ -231,7 +231,8 @@ def test_omega_ema_kernel_forms(gpu, num_kv, kv_groups, max_blocks, adjacent):
     np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-7)
 
 
-@pytest.mark.parametrize("num_kv,kv_groups,max_blocks", [(2, 4, 512), (2, 4, 513), (1, 9, 768), (3, 1, 1025), (1, 2, 20000)])
+@pytest.mark.parametrize("num_kv,kv_groups,max_blocks", [(3, 4, 1), (2, 8, 65), (2, 5, 256), (2, 4, 257), (2, 4, 512), (2, 4, 513),
+                                                         (1, 9, 768), (3, 1, 1025), (1, 2, 20000)])
 def test_omega_ema_one_and_two_kernels(gpu, num_kv, kv_groups, max_blocks):
     # the form with a workspace (chunks of 256 pages: a whole last one, one
     # page more, more chunks than lanes) and the one without agree with the
