@@ -104,15 +104,15 @@ def clone_pool(pool: ops.PagedPool) -> ops.PagedPool:
 # KiB) and WRITE_SIZE all of them (262144 KiB), hence the factor 2.  Measured
 # with `bench.py --calibrate` under rocprofv3 --pmc (summary and commands in
 # profiles/decode_config2_hbm_traffic.txt); re-measured when the kernel changes.
-TRAFFIC_BYTES = {(2, "default"): 86515541}
+TRAFFIC_BYTES = {(2, "default"): 86607087}
 
 # encode_pages_kernel at config 3, from rocprofv3 --pmc on MI355X
 # (profiles/encode_config3_counters.txt): VALU instructions per launch (MFMA
 # included) and HBM bytes (FETCH_SIZE * 2 + WRITE_SIZE).  The VALU-issue bound
 # is that count at one wave64 VALU instruction per 4 cycles on each of the
 # 1024 SIMDs at 2.4 GHz.
-ENCODE_VALU_INSTS = {3: 7061123}
-ENCODE_TRAFFIC_BYTES = {3: 55632656}
+ENCODE_VALU_INSTS = {3: 5177707}
+ENCODE_TRAFFIC_BYTES = {3: 56232111}
 # HBM bytes per Mode-A decode (modea_fast_kernel, page_size 16; profiles/
 # modea_config2shape_counters.txt) and per fused_decode_ragged step (both
 # tiers' ragged_pipe_kernel launches; profiles/ragged_config2_hbm_traffic.txt),

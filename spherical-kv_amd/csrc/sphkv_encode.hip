@@ -566,8 +566,8 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
 // load, so the rate is the workgroups resident: three per CU at 80 VGPRs and
 // 31 KB of LDS (fp32 keys: two).  Eight waves per SIMD (64 VGPRs) spill: 462
 // us against 315 for the 98,000-token batch below.  Measured (per launch): 16
-// prompts of 500..12,000 tokens 254 -> 186 us (3.7 TB/s of traffic), 8,192
-// tokens 26.7 -> 25, the same tokens' codes at three tiers 46.5 -> 29.
+// prompts of 500..12,000 tokens 254 -> 188 us (3.7 TB/s of traffic), 8,192
+// tokens 26.7 -> 22.8, the same tokens' codes at three tiers 43.4 -> 26.7.
 template <int DH, bool K32, bool CODES>
 __global__ __launch_bounds__(kEncWaves * 64) __attribute__((amdgpu_waves_per_eu(6, 6))) void encode_pages_kernel(EncodeArgs a) {
   using L = EncodeLds<DH, K32>;

@@ -1173,7 +1173,7 @@ __global__ __launch_bounds__(256) void omega_ema_kernel(OmegaLaunch a) {
 // l directly follows m, as in partial_scratch; no load for q heads past
 // kv_groups), the group's maxima and sums reduced together.  Same formula as
 // omega_ema_kernel.  Up to 256 blocks NT is 256: the chain of barriers and
-// shuffles is what such a call costs, and 4 waves pass it sooner than 16 (16
+// shuffles is what such a call costs, and 4 waves pass it sooner than 16 (8
 // kv heads, 64 blocks: 7.0 -> 4.0 us).
 template <int PPT, int KG, int NT>
 __global__ __launch_bounds__(NT) void omega_ema_fast_kernel(OmegaLaunch a, int adjacent) {

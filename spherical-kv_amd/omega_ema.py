@@ -43,14 +43,16 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
         out = torch.empty_like(omega_prev)
     elif out.dtype != torch.float32 or not out.is_contiguous() or out.shape != omega_prev.shape:
         raise ValueError("out must be a contiguous fp32 tensor shaped like omega_prev")
-    args = (m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(), out.data_ptr(),
-            int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta))
-    if args[8] > 512:                                    # long tables: two kernels over scratch of this call's stream
-        nws = _lib.sphkv_omega_ema_workspace_bytes(*args[6:9])
-        ws = torch.empty(max(nws, 8), dtype=torch.uint8, device=out.device)
-        rc = _lib.sphkv_omega_ema_ws(*args, ws.data_ptr(), max(nws, 8), sphkv_lib.current_stream())
-    else:
-        rc = _lib.sphkv_omega_ema(*args, sphkv_lib.current_stream())
+    if max_blocks <= 512:
+        rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(),
+                                  out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),
+                                  sphkv_lib.current_stream())
+    else:                                                # long tables: two kernels over scratch of this call's stream
+        nws = max(_lib.sphkv_omega_ema_workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks)), 8)
+        ws = torch.empty(nws, dtype=torch.uint8, device=out.device)
+        rc = _lib.sphkv_omega_ema_ws(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1),
+                                     omega_prev.data_ptr(), out.data_ptr(), int(num_kv), int(kv_groups),
+                                     int(max_blocks), float(ema_beta), ws.data_ptr(), nws, sphkv_lib.current_stream())
     check(rc, "omega_ema")
     return out
 
