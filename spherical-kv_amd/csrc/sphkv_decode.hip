@@ -1113,8 +1113,9 @@ __global__ __launch_bounds__(256) void decode_merge_kernel(const float* __restri
 // ---------------------------------------------------------------------------
 // Decode-time tail of the Mode-B step (spherical_kv_pipeline.py:2248-2342,
 // 2389-2475).  One 256-thread workgroup per (sequence, kv head) sh and slice
-// of up to 128 floats of its GQA*DH output (the slice's q heads' tail logits,
-// the log-sum-exp of the slice's columns); slice 0 also appends.  The tail
+// of up to 128 floats (tail_slice: 512 with many sequences) of its GQA*DH
+// output (the slice's q heads' tail logits, the log-sum-exp of the slice's
+// columns); slice 0 also appends.  The tail
 // counts come in two copies: a step reads copy `parity` and an appending
 // step writes the other, so the slices of one sh never see each other's
 // update.

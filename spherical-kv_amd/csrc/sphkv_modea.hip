@@ -1115,7 +1115,8 @@ namespace sphkv {
 // 952-987): per q head, pages with l > 0 compete in a softmax of their (m, l)
 // -- w = exp(max(m - max_p m, -60)) * l, mass = w / max(sum w, 1e-12) -- the
 // masses are averaged over each kv head's q heads and blended into omega:
-// omega' = omega * beta + mass * (1 - beta).  One workgroup per kv head.
+// omega' = omega * beta + mass * (1 - beta).  One workgroup per kv head, or
+// (a workspace, past kOmegaSplitBlocks blocks) one per 256 pages of a q head.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) {
   for (int o = 32; o >= 1; o >>= 1) {

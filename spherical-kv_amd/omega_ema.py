@@ -48,11 +48,13 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
                                   out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),
                                   sphkv_lib.current_stream())
     else:                                                # long tables: two kernels over scratch of this call's stream
-        nws = max(_lib.sphkv_omega_ema_workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks)), 8)
-        ws = torch.empty(nws, dtype=torch.uint8, device=out.device)
+        # sphkv_omega_ema_workspace_bytes: a pair per (q head, 256 blocks) and per (q head, block)
+        n = 2 * nq * (int(max_blocks) + (int(max_blocks) + 255) // 256)
+        ws = m_q.new_empty(n)
         rc = _lib.sphkv_omega_ema_ws(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1),
                                      omega_prev.data_ptr(), out.data_ptr(), int(num_kv), int(kv_groups),
-                                     int(max_blocks), float(ema_beta), ws.data_ptr(), nws, sphkv_lib.current_stream())
+                                     int(max_blocks), float(ema_beta), ws.data_ptr(), 4 * n,
+                                     sphkv_lib.current_stream())
     check(rc, "omega_ema")
     return out
 
