@@ -194,7 +194,7 @@ def test_encode_non_unit_codebooks_bit_exact(gpu, kind):
 def test_encode_small_gaps_scales_and_bit_patterns(gpu, dh, H, L, fp32):
     # the MFMA ranking and its exact pass: gaps of 1e-7 to 1e-2 between the two
     # best centroids (around the slack past which the ranking stands), ties of
-    # three centroids, groups from fp16 denormals to large, pages of every
+    # three centroids, groups from zero and fp16 denormals to large, pages of every
     # tier mixed in one workgroup, missing rows at the end of a workgroup; V and
     # dense K of any bit pattern (negative zeros, infinities, NaNs) as they are
     rng = np.random.default_rng(dh + fp32)
@@ -213,7 +213,8 @@ def test_encode_small_gaps_scales_and_bit_patterns(gpu, dh, H, L, fp32):
                 a, b, c = rng.choice(C, size=3, replace=False)
                 eps = np.float32(10.0 ** rng.uniform(-7, -2))
                 v = cb[j, a] + cb[j, b] * (1 - eps) + (cb[j, c] * (1 - eps) if t % 3 == 0 else 0)
-                K[h, t, j * g:(j + 1) * g] = v * np.float32(2.0 ** rng.integers(-22, 9))
+                scale = np.float32(2.0 ** rng.integers(-22, 9)) if (t + j) % 13 else np.float32(0)   # 0 (and -0): a zero key
+                K[h, t, j * g:(j + 1) * g] = v * scale
     dense = np.stack([t == fmt.DENSE_TIER_ID for t in tier_of])
     if fp32:
         K[dense] = np.where(np.isnan(K[dense]), 1.0, K[dense])       # (a NaN's payload is not kept by the conversion)
