@@ -604,6 +604,13 @@ int sphkv_plan_pages_fill(const uint8_t* tier_of, int64_t tier_stride, const int
  * * slots_per_cu; otherwise max(8, ceil(total / (4 * num_cus *
  * slots_per_cu))).  Returns r >= 8, or a negative SPHKV_E* code.
  *
+ * sphkv_work_pool_rows_per_item: rows per item of a pool's own list: the
+ * above at one slot per CU, or the smallest r >= 64 whose items run in three
+ * rounds (r >= 64 of the above with more than 3 * num_cus ranges), whichever
+ * bounds the step's time lower: an item costs its CU about 30 rows more than
+ * it holds, and the step ends at most its longest item after the CUs' mean
+ * load.  Returns r >= 8, or a negative SPHKV_E* code.
+ *
  * sphkv_work_fill: work int32 [n, 4] = (sh, first_row, end_row, stride) with
  * n = sum_i max(1, ceil(len_i / rows_per_item)) (capacity max_items), and
  * work_start int32 [num_sh + 1] = first item of each range.  interleave != 0:
@@ -612,6 +619,7 @@ int sphkv_plan_pages_fill(const uint8_t* tier_of, int64_t tier_stride, const int
  * a negative SPHKV_E* code.
  */
 int32_t sphkv_work_rows_per_item(const int32_t* row_start, int32_t num_sh, int32_t num_cus, int32_t slots_per_cu);
+int32_t sphkv_work_pool_rows_per_item(const int32_t* row_start, int32_t num_sh, int32_t num_cus);
 int64_t sphkv_work_fill(const int32_t* row_start, int32_t num_sh, int32_t rows_per_item, int32_t interleave,
                         int32_t* work, int64_t max_items, int32_t* work_start);
 

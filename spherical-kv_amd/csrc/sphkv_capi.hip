@@ -60,6 +60,41 @@ int64_t work_items(const int32_t* rs, int32_t num_sh, int64_t r) {
   return n;
 }
 
+// smallest rows per item whose items fit `target` (at least 8 and the mean),
+// or about four items per target slot where the ranges alone are more
+int32_t rows_per_item(const int32_t* rs, int32_t num_sh, int64_t target) {
+  const int64_t total = num_sh > 0 ? (int64_t)rs[num_sh] - rs[0] : 0;
+  if (total == 0) return 8;
+  int64_t max_len = 0;
+  for (int32_t i = 0; i < num_sh; ++i) max_len = std::max<int64_t>(max_len, (int64_t)rs[i + 1] - rs[i]);
+  int64_t lo = std::max<int64_t>(8, (total + target - 1) / target), hi = std::max(lo, max_len);
+  if (work_items(rs, num_sh, hi) > target) return (int32_t)std::max<int64_t>(8, (total + 4 * target - 1) / (4 * target));
+  // the item total does not grow with r: the first r in [lo, hi] that fits
+  while (lo < hi) {
+    const int64_t mid = lo + (hi - lo) / 2;
+    if (work_items(rs, num_sh, mid) <= target) hi = mid; else lo = mid + 1;
+  }
+  return (int32_t)lo;
+}
+
+// Rows a CU decodes in the time that one more work item costs it (6.5 us:
+// prologue and merge).
+constexpr double kItemRows = 30;
+
+// Longest time of a step over items of at most r rows, in rows of one CU: the
+// dispatcher hands items out as CUs free up, so none starts its last one
+// later than the mean load, and that takes the longest item's time more.  One
+// round takes the longest item.
+double step_rows(const int32_t* rs, int32_t num_sh, int32_t num_cus, double per_cu, int64_t r) {
+  int64_t longest = 0;
+  for (int32_t i = 0; i < num_sh; ++i) {
+    const int64_t len = (int64_t)rs[i + 1] - rs[i], n = len > r ? (len + r - 1) / r : 1;
+    longest = std::max(longest, (len + n - 1) / n);
+  }
+  const int64_t items = work_items(rs, num_sh, r);
+  return items <= num_cus ? longest + kItemRows : per_cu + kItemRows * items / num_cus + longest;
+}
+
 bool dh_ok(int32_t dh) { return dh == 64 || dh == 128; }
 bool gqa_ok(int32_t g) { return g == 1 || g == 2 || g == 4 || g == 8; }
 
@@ -952,21 +987,24 @@ int32_t sphkv_work_rows_per_item(const int32_t* row_start, int32_t num_sh, int32
   if (num_cus < 1 || slots_per_cu < 1) return fail(SPHKV_EINVAL, "%s: num_cus and slots_per_cu must be >= 1", fn);
   if (!row_start_ok(row_start, num_sh))
     return fail(SPHKV_EINVAL, "%s: row_start must hold num_sh + 1 non-decreasing rows >= 0", fn);
-  const int64_t total = num_sh > 0 ? (int64_t)row_start[num_sh] - row_start[0] : 0;
-  if (total == 0) { ok(); return 8; }
-  const int64_t target = (int64_t)num_cus * slots_per_cu;
-  int64_t max_len = 0;
-  for (int32_t i = 0; i < num_sh; ++i) max_len = std::max<int64_t>(max_len, (int64_t)row_start[i + 1] - row_start[i]);
-  int64_t lo = std::max<int64_t>(8, (total + target - 1) / target), hi = std::max(lo, max_len);
   ok();
-  // more ranges than one item per CU covers: about four smaller items per CU
-  if (work_items(row_start, num_sh, hi) > target) return (int32_t)std::max<int64_t>(8, (total + 4 * target - 1) / (4 * target));
-  // the item total does not grow with r: the first r in [lo, hi] that fits
-  while (lo < hi) {
-    const int64_t mid = lo + (hi - lo) / 2;
-    if (work_items(row_start, num_sh, mid) <= target) hi = mid; else lo = mid + 1;
-  }
-  return (int32_t)lo;
+  return rows_per_item(row_start, num_sh, (int64_t)num_cus * slots_per_cu);
+}
+
+int32_t sphkv_work_pool_rows_per_item(const int32_t* row_start, int32_t num_sh, int32_t num_cus) {
+  const char* fn = "sphkv_work_pool_rows_per_item";
+  if (num_cus < 1) return fail(SPHKV_EINVAL, "%s: num_cus must be >= 1", fn);
+  if (!row_start_ok(row_start, num_sh))
+    return fail(SPHKV_EINVAL, "%s: row_start must hold num_sh + 1 non-decreasing rows >= 0", fn);
+  ok();
+  const int32_t one = rows_per_item(row_start, num_sh, num_cus);
+  if (num_sh < 1) return one;
+  const double per_cu = ((double)row_start[num_sh] - row_start[0]) / num_cus;
+  // One round already near the mean: more items, each longer than half of r >=
+  // 64 rows, take at least per_cu + kItemRows + 32.
+  if (num_sh <= num_cus && one <= per_cu + 32) return one;
+  const int32_t few = std::max(64, num_sh > (int64_t)3 * num_cus ? one : rows_per_item(row_start, num_sh, (int64_t)3 * num_cus));
+  return step_rows(row_start, num_sh, num_cus, per_cu, few) <= step_rows(row_start, num_sh, num_cus, per_cu, one) ? few : one;
 }
 
 int64_t sphkv_work_fill(const int32_t* row_start, int32_t num_sh, int32_t rows_per_item, int32_t interleave,

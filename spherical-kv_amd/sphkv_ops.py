@@ -62,40 +62,28 @@ def auto_rows_per_item(row_start: np.ndarray, num_cus: int, slots_per_cu: int = 
     running at once; at least 8 rows).  When there are more ranges than that
     (each needs an item of its own), about four smaller items per CU, which
     the dispatcher balances as CUs free up."""
-    return _rows_per_item(_row_start32(row_start), num_cus, slots_per_cu)
-
-
-def _rows_per_item(rs: np.ndarray, num_cus: int, slots_per_cu: int) -> int:
+    rs = _row_start32(row_start)
     r = load().sphkv_work_rows_per_item(rs.ctypes.data, rs.size - 1, int(num_cus), int(slots_per_cu))
     check(min(r, 0), "sphkv_work_rows_per_item")
     return int(r)
 
 
-ITEM_ROWS = 30           # rows a CU decodes in the time that one more work item costs it (6.5 us)
-
-
 def pool_rows_per_item(row_start: np.ndarray, num_cus: int) -> int:
-    """Rows per work item of a pool's own list: auto_rows_per_item's one item
-    per CU while that is balanced, else (uneven ranges, or more ranges than
-    CUs) the smallest items of at least 64 rows that run in three rounds.  An
-    item costs its CU a prologue and a merge worth ITEM_ROWS rows, so short
-    contexts want few items: 64 sequences of 150..2100 tokens (512 ranges) take
-    59.1 us per step as 1,264 items, 52.8 as 768, 54.0 as 512 and 58.1 as 816
-    (a fourth round); 64 of 300..600 40.7 as 1,224, 27.9 as 512; 26 of 200..
-    16,000 (208 ranges) 130.8 as 256, 118.0 as 464.  Past 400 rows per CU the
-    prologues no longer count and auto_rows_per_item's smaller items balance
-    better (64 of 2K..32K: 523 us as 1,264 items, 551 as 760)."""
+    """Rows per work item of a pool's own list (library routine
+    sphkv_work_pool_rows_per_item): auto_rows_per_item's items, or fewer and
+    larger ones that run in three rounds, whichever bounds the step lower.  An
+    item costs its CU a prologue and a merge worth 30 rows, so short contexts
+    want few items: 64 sequences of 150..2100 tokens (512 ranges) take 59.1 us
+    per step as 1,264 items, 52.8 as 768, 54.0 as 512 and 58.1 as 816 (a fourth
+    round); 64 of 300..600 40.7 as 1,224, 27.9 as 512; 26 of 200..16,000 (208
+    ranges) 130.8 as 256, 118.0 as 464.  Where the prologues count for little,
+    smaller items balance better (64 of 2K..32K: 523 us as 1,264 items, 551 as
+    760), and near three ranges per CU three rounds leave none to split a long
+    sequence with."""
     rs = _row_start32(row_start)
-    num_sh, per_cu = rs.size - 1, (int(rs[-1]) - int(rs[0])) / num_cus
-    one = _rows_per_item(rs, num_cus, 1)
-    if num_sh <= num_cus:
-        if one <= per_cu + 2 * ITEM_ROWS + 32:         # the comparison below, at the smallest possible three
-            return one
-        three = max(64, _rows_per_item(rs, num_cus, 3))
-        return three if per_cu + 3 * ITEM_ROWS + three / 2 < one + ITEM_ROWS else one
-    if per_cu > 400:
-        return one
-    return max(64, one if num_sh > 3 * num_cus else _rows_per_item(rs, num_cus, 3))
+    r = load().sphkv_work_pool_rows_per_item(rs.ctypes.data, rs.size - 1, int(num_cus))
+    check(min(r, 0), "sphkv_work_pool_rows_per_item")
+    return int(r)
 
 
 def _work_fill(rs: np.ndarray, rows_per_item: int, interleave: bool, buf_ptr: int, head: int, cap: int) -> int:

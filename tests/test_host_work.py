@@ -138,3 +138,58 @@ def test_pool_rows_per_item_is_bounded(num_sh):
     rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
     n, n1 = (_items(lens, f(rs, 256)) for f in (ops.pool_rows_per_item, ops.auto_rows_per_item))
     assert n <= max(768, num_sh, n1)
+
+
+def _step_model(lens, r, num_cus=256, item_rows=30):
+    """Rows that a CU spends on the step's critical path: items handed out in
+    list order to the first free CU, each costing item_rows more than it holds."""
+    import heapq
+    free = [0] * num_cus
+    for n in lens:
+        k = max(1, -(-int(n) // r))
+        for i in range(k):
+            heapq.heapreplace(free, free[0] + (int(n) + k - 1 - i) // k + item_rows)
+    return max(free)
+
+
+@pytest.mark.parametrize("num_sh,few,base,long", [
+    (768, 8, 13, 6250), (768, 8, 20, 8192), (760, 8, 13, 2000), (768, 16, 13, 2000), (768, 8, 32, 2048), (736, 8, 13, 6250),
+    (704, 8, 13, 6250), (776, 8, 13, 6250), (512, 8, 36, 6250), (276, 16, 40, 4000), (800, 8, 100, 1000), (250, 8, 13, 6250),
+])
+def test_pool_rows_per_item_splits_long_sequences(num_sh, few, base, long):
+    # one or two long sequences among many short ones: the step is as short as
+    # with auto_rows_per_item's items (5 %: the model's rounding of one item)
+    lens = np.full(num_sh, base)
+    lens[num_sh // 3:num_sh // 3 + few] = long
+    rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    r, auto = ops.pool_rows_per_item(rs, 256), ops.auto_rows_per_item(rs, 256)
+    assert _step_model(lens, r) <= 1.05 * _step_model(lens, auto)
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_pool_rows_per_item_is_no_worse_than_one_item_per_cu(seed):
+    rng = np.random.default_rng(seed)
+    for _ in range(40):
+        num_sh = int(rng.integers(200, 850))
+        lens = np.exp(rng.uniform(np.log(4), np.log(rng.choice([40, 300, 2000])), size=num_sh)).astype(int)
+        lens[rng.choice(num_sh, 8 * int(rng.integers(0, 3)), replace=False)] = int(rng.choice([400, 2000, 8000]))
+        rs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        r, auto = ops.pool_rows_per_item(rs, 256), ops.auto_rows_per_item(rs, 256)
+        n, n_auto, mean = _items(lens, r), _items(lens, auto), lens.sum() / 256
+        longest, longest_auto = min(r, lens.max()), min(auto, lens.max())
+        assert max(mean + 30 * n / 256, longest + 30) <= 1.05 * max(mean + 30 * n_auto / 256, longest_auto + 30)
+        assert _step_model(lens, r) <= 1.08 * _step_model(lens, auto)
+
+
+def test_pool_rows_per_item_of_uneven_batches():
+    # 64 sequences of 150..2100 and of 2K..32K tokens, 26 of 200..16,000, 16
+    # of 500..12,000 and one of 32K, 8 kv heads each
+    def lens(n, lo, hi):
+        at = [lo + int((hi - lo) * ((i * 0.6180339887498949 + 0.5) % 1.0)) for i in range(n)]
+        return np.repeat([-(-t // 16) for t in at], 8)
+    for args, items in (((64, 150, 2100), 768), ((64, 2048, 32768), 1272), ((26, 200, 16000), 768), ((16, 500, 12000), 256)):
+        x = lens(*args)
+        rs = np.concatenate([[0], np.cumsum(x)]).astype(np.int64)
+        assert _items(x, ops.pool_rows_per_item(rs, 256)) == items, args
+    with pytest.raises(Exception, match="num_cus"):
+        ops.pool_rows_per_item(np.array([0, 10]), 0)
