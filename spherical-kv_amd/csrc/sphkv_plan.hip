@@ -126,18 +126,19 @@ __device__ __forceinline__ int32_t* ch_rec(const PlanLaunch& a, int sh, int c) {
 }
 
 // Tier slots of the thread's tokens t0 + threadIdx.x + 256 i < t1 of a chunk
-// (-1 past it), their bytes all in flight together.
+// (-1 past it), their bytes all in flight together.  A chunk past the sequence's
+// end reads nothing: a row may be only its sequence long.
 __device__ __forceinline__ void load_tiers(const PlanLaunch& a, int sh, int t0, int t1, int (&k)[kPlanIters]) {
   const uint8_t* t_of = a.tier_of + (int64_t)sh * a.tier_stride;
   int raw[kPlanIters];
-  if (t0 >= a.max_len) {                                 // max_len 0: the rows are empty
+  if (t0 >= t1) {                                        // workgroup-uniform
     for (int it = 0; it < kPlanIters; ++it) k[it] = -1;
     return;
   }
 #pragma unroll
   for (int it = 0; it < kPlanIters; ++it) {
     const int t = t0 + it * kPlanThreads + (int)threadIdx.x;
-    raw[it] = t_of[t < t1 ? t : t0];                     // t0 < max_len, the row's width
+    raw[it] = t_of[t < t1 ? t : t0];
   }
 #pragma unroll
   for (int it = 0; it < kPlanIters; ++it) k[it] = t0 + it * kPlanThreads + (int)threadIdx.x < t1 ? tier_slot(raw[it]) : -1;

@@ -190,3 +190,34 @@ def test_device_plan_chunk_lengths(gpu, lengths, num_kv):
     dp = ops.plan_pages_gpu(t, lens, num_kv, 64, row_base=torch.from_numpy(base).to(gpu))
     log(f"chunk lengths: {len(tier_of)} ranges of up to {max(lengths)}: rows {dp.rows}")
     _check(dp, tier_of, lengths, num_kv, base)
+
+
+@pytest.mark.parametrize("lengths,num_kv,max_len", [([4000, 5], 1, 4000), ([3000, 0], 2, 3000), ([700, 1], 4, 9000)])
+def test_device_plan_reads_no_row_past_its_length(gpu, lengths, num_kv, max_len):
+    # the header's contract at the C entry points: only the first lens[s]
+    # entries of a row are read, so the last row may end with its sequence
+    # (here also inside rows filled with invalid ids past their lengths)
+    lib = ops.load()
+    rng = np.random.default_rng(max_len)
+    num_sh, dh = len(lengths) * num_kv, 64
+    rows = [rng.choice(np.array([0, 1, 2, 3, 0xFF], np.uint8), size=L) for L in lengths for _ in range(num_kv)]
+    flat = np.full((num_sh - 1) * max_len + lengths[-1], 7, np.uint8)
+    for sh, r in enumerate(rows):
+        flat[sh * max_len:sh * max_len + r.size] = r
+    tier_of = torch.from_numpy(flat).to(gpu)
+    lens = torch.tensor(lengths, dtype=torch.int32, device=gpu)
+    work = torch.empty(lib.sphkv_plan_pages_work_ints(len(lengths), num_kv, max_len), dtype=torch.int32, device=gpu)
+    row_start, totals = (torch.empty(n, dtype=torch.int32, device=gpu) for n in (num_sh + 1, 4))
+    log(f"plan rows end with their sequences: {lengths} x {num_kv}, max_len {max_len}")
+    assert lib.sphkv_plan_pages_count(tier_of.data_ptr(), max_len, lens.data_ptr(), len(lengths), num_kv, max_len, dh,
+                                      work.data_ptr(), work.numel(), row_start.data_ptr(), totals.data_ptr(), ops._stream()) == 0
+    n, nbytes, bad, ovf = totals.cpu().tolist()
+    want = fmt.plan_pages([r.astype(np.int32) for r in rows], None, len(lengths), num_kv, dh, 16)
+    assert (n, bad, ovf) == (want.num_rows, 0, 0) and (row_start.cpu().numpy() == want.row_start).all()
+    b32 = torch.full((n * 23,), -9, dtype=torch.int32, device=gpu)
+    tokens = torch.full((n, 16), -9, dtype=torch.int64, device=gpu)
+    at = [b32.data_ptr() + 4 * n * i for i in (0, 1, 2, 5, 6, 7)]
+    assert lib.sphkv_plan_pages_fill(tier_of.data_ptr(), max_len, lens.data_ptr(), None, 0, None, len(lengths), num_kv, max_len,
+                                     dh, work.data_ptr(), n, at[0], at[1], at[2], at[3], at[4], tokens.data_ptr(), at[5],
+                                     None, ops._stream()) == 0
+    assert (tokens.cpu().numpy() == want.tokens).all() and (b32[:n].cpu().numpy() == want.tier).all()
