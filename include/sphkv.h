@@ -565,7 +565,8 @@ int sphkv_build_layer_pool(const float* r, const int32_t* theta, int64_t n_elems
  * lens[s] <= max_len <= tier_stride for every sequence; tokens are
  * processed in chunks, max_len sizes the grid.  The workspace holds
  * sphkv_plan_pages_work_ints(num_seqs, num_kv, max_len) int32 and carries
- * the counts from phase 1 to phase 2 (same arguments in both).
+ * the counts from phase 1 to phase 2 (same arguments in both); one sized for
+ * the largest arguments serves all smaller ones.
  *
  * Phase 1, sphkv_plan_pages_count: row_start int32
  * [num_seqs * num_kv + 1]; totals int32 [4] receives (rows, byte-pool size

@@ -40,6 +40,8 @@
 //   plan_fill_kernel   per (sequence, head, chunk): its share of the page
 //                      rows, then each token's rank within its tier (chunk
 //                      base + wave ballots) puts it in its page slot
+#include <algorithm>
+
 #include "sphkv_common.h"
 #include "sphkv_internal.h"
 
@@ -437,10 +439,15 @@ __global__ __launch_bounds__(kPlanThreads) void plan_fill_kernel(PlanLaunch a) {
   }
 }
 
+// Enough for these sizes and for all smaller ones, so that a workspace sized
+// once for the largest prompt serves the others (a shorter prompt may take the
+// short chunks: at most `most` of them).
 int64_t plan_work_ints(int num_sh, int max_len) {
-  const int chunk = plan_chunk(num_sh, max_len);
-  const int64_t nch = max_len <= 0 ? 1 : ((int64_t)max_len + chunk - 1) / chunk;
-  return (int64_t)num_sh * kRec + (int64_t)num_sh * nch * kChRec;
+  const int64_t len = max_len <= 0 ? 1 : max_len;
+  const int64_t most = (int64_t)kPlanFewChunks * (kPlanChunk / kPlanChunkShort);
+  const int64_t longer = num_sh * ((len + kPlanChunk - 1) / kPlanChunk);
+  const int64_t shorter = num_sh * ((len + kPlanChunkShort - 1) / kPlanChunkShort);
+  return (int64_t)num_sh * kRec + std::max(longer, std::min(shorter, most)) * kChRec;
 }
 
 int launch_plan(const PlanLaunch& L0, int phase, hipStream_t stream) {

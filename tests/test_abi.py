@@ -254,6 +254,26 @@ def test_noalloc_refuses_work_beyond_its_scratch():
     assert lib.sphkv_decode_paged_noalloc(*args) == 0
 
 
+def test_plan_pages_workspace_of_the_largest_prompt_serves_the_others():
+    # one workspace for every smaller call: the size grows with each argument,
+    # and the count entry takes it at any smaller size (the chunk length that
+    # the planner picks changes with the sizes)
+    lib = sphkv_lib.load()
+    ints = lib.sphkv_plan_pages_work_ints
+    lens = [0, 1, 511, 512, 513, 2048, 2049, 8192, 8193, 16384, 65536, 65537, 524288, 524289, 2 ** 31 - 1]
+    for seqs, kv in ((1, 1), (1, 8), (8, 8), (16, 8), (31, 8), (32, 8), (33, 8), (300, 4)):
+        sizes = [ints(seqs, kv, n) for n in lens]
+        assert sizes == sorted(sizes)
+        assert all(ints(seqs + 1, kv, n) >= s for n, s in zip(lens, sizes))
+        for n in lens:
+            rc = lib.sphkv_plan_pages_count(None, lens[-1], None, seqs, kv, n, 64, None, sizes[-1], None, None, None)
+            assert rc == -1 and "null pointer" in lib.sphkv_last_error().decode()
+    assert lib.sphkv_plan_pages_count(None, 8192, None, 8, 8, 8192, 64, None, ints(8, 8, 16384), None, None, None) == -1
+    assert "null pointer" in lib.sphkv_last_error().decode()
+    assert lib.sphkv_plan_pages_count(None, 8192, None, 8, 8, 8192, 64, None, 64, None, None, None) == -1
+    assert "workspace too small" in lib.sphkv_last_error().decode()
+
+
 def test_decode_plan_argument_errors():
     import ctypes
     lib = sphkv_lib.load()
