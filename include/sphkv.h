@@ -527,8 +527,9 @@ int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_
  * what it wants (0: none, one kernel is as fast; negative on bad sizes), and
  * with that many bytes (8-byte aligned, contents irrelevant, free again when
  * the call has run) the pages are read by workgroups of 256 instead of one per
- * kv head.  workspace NULL: as sphkv_omega_ema.  Calls that share a workspace
- * must not run concurrently.
+ * kv head.  workspace NULL, or a table that wants none (any workspace is taken
+ * and left alone): as sphkv_omega_ema.  Calls that share a workspace must not
+ * run concurrently.
  */
 int64_t sphkv_omega_ema_workspace_bytes(int32_t num_kv, int32_t kv_groups, int32_t max_blocks);
 int sphkv_omega_ema_ws(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,

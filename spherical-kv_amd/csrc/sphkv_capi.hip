@@ -884,15 +884,17 @@ static int omega_ema(const char* fn, const float* m_q, const float* l_q, int64_t
     return fail(SPHKV_EINVAL, "%s: kv_groups must be 1..%d", fn, sphkv::kOmegaMaxGroups);
   if (q_stride < 0 || page_stride < 0) return fail(SPHKV_EINVAL, "%s: negative stride", fn);
   if (num_kv == 0 || max_blocks == 0) return ok();
-  if (!m_q || !l_q || !omega_prev || !omega_out) return fail(SPHKV_EINVAL, "%s: null pointer argument", fn);
-  sphkv::OmegaLaunch L{m_q, l_q, q_stride, page_stride, omega_prev, omega_out, num_kv, kv_groups, max_blocks,
-                       ema_beta, nullptr};
-  if (ws) {
+  // (a short table runs in one kernel, whatever workspace is offered)
+  const bool split = ws && max_blocks > sphkv::kOmegaSplitBlocks &&
+                     (int64_t)num_kv * kv_groups * ((max_blocks + 255) / 256) < ((int64_t)1 << 31);
+  if (split) {
     const int64_t need = 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
     if (ws_bytes < need || ((uintptr_t)ws & 7) != 0)
       return fail(SPHKV_EINVAL, "%s: workspace needs %lld bytes, 8-byte aligned", fn, (long long)need);
-    if ((int64_t)num_kv * kv_groups * ((max_blocks + 255) / 256) < ((int64_t)1 << 31)) L.ws = static_cast<float*>(ws);
   }
+  if (!m_q || !l_q || !omega_prev || !omega_out) return fail(SPHKV_EINVAL, "%s: null pointer argument", fn);
+  const sphkv::OmegaLaunch L{m_q, l_q, q_stride, page_stride, omega_prev, omega_out, num_kv, kv_groups, max_blocks,
+                             ema_beta, split ? static_cast<float*>(ws) : nullptr};
   return launch_status(sphkv::launch_omega(L, (hipStream_t)stream), fn);
 }
 

@@ -10,6 +10,7 @@ place).  One HIP kernel (two past 512 blocks); raises if libsphkv.so is missing.
 """
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -20,6 +21,11 @@ from sphkv_lib import check
 _lib = sphkv_lib.load()
 
 EMA_BETA = 0.9          # spherical_kv_pipeline.py EMA_BETA
+
+
+@lru_cache(maxsize=256)
+def _workspace_bytes(num_kv: int, kv_groups: int, max_blocks: int) -> int:
+    return _lib.sphkv_omega_ema_workspace_bytes(num_kv, kv_groups, max_blocks)
 
 
 def _view_ok(t: torch.Tensor, name: str) -> None:
@@ -43,17 +49,16 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
         out = torch.empty_like(omega_prev)
     elif out.dtype != torch.float32 or not out.is_contiguous() or out.shape != omega_prev.shape:
         raise ValueError("out must be a contiguous fp32 tensor shaped like omega_prev")
-    if max_blocks <= 512:
+    need = _workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks))
+    if need <= 0:                                        # one kernel (and, for bad sizes, the call's own error)
         rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(),
                                   out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),
                                   sphkv_lib.current_stream())
     else:                                                # long tables: two kernels over scratch of this call's stream
-        # sphkv_omega_ema_workspace_bytes: a pair per (q head, 256 blocks) and per (q head, block)
-        n = 2 * nq * (int(max_blocks) + (int(max_blocks) + 255) // 256)
-        ws = m_q.new_empty(n)
+        ws = m_q.new_empty(need // 4)
         rc = _lib.sphkv_omega_ema_ws(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1),
                                      omega_prev.data_ptr(), out.data_ptr(), int(num_kv), int(kv_groups),
-                                     int(max_blocks), float(ema_beta), ws.data_ptr(), 4 * n,
+                                     int(max_blocks), float(ema_beta), ws.data_ptr(), need,
                                      sphkv_lib.current_stream())
     check(rc, "omega_ema")
     return out

@@ -240,6 +240,25 @@ def test_omega_ema_argument_errors():
     assert lib.sphkv_omega_ema(None, None, 130, 2, None, None, 8, 4, 0, 0.9, None) == 0
 
 
+def test_omega_ema_workspace_query_and_call_agree():
+    # what the size query names is what the call takes: 0 bytes for the tables
+    # that it says want none, whatever pointer comes with them
+    lib = sphkv_lib.load()
+    ws = ctypes.create_string_buffer(64)
+    at = (ctypes.addressof(ws) + 7) & ~7
+    for kv, g, n in ((8, 4, 1), (8, 4, 512), (8, 4, 513), (1, 8, 4096), (2, 9, 5000)):
+        need = lib.sphkv_omega_ema_workspace_bytes(kv, g, n)
+        assert need >= 0
+        for size, msg in ((need, "null pointer"),) + (((need - 1, "workspace needs"),) if need else ()):
+            assert lib.sphkv_omega_ema_ws(None, None, 130, 2, None, None, kv, g, n, 0.9, at, size, None) == -1
+            assert msg in lib.sphkv_last_error().decode()
+        if need:
+            assert lib.sphkv_omega_ema_ws(None, None, 130, 2, None, None, kv, g, n, 0.9, at + 4, need, None) == -1
+            assert "8-byte aligned" in lib.sphkv_last_error().decode()
+    assert lib.sphkv_omega_ema_workspace_bytes(8, 4, 512) == 0
+    assert lib.sphkv_omega_ema_workspace_bytes(8, 0, 512) < 0 and lib.sphkv_omega_ema_workspace_bytes(-1, 4, 512) < 0
+
+
 def test_noalloc_refuses_work_beyond_its_scratch():
     # the size check runs before any device access
     lib = sphkv_lib.load()

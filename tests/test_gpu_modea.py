@@ -256,3 +256,20 @@ def test_omega_ema_one_and_two_kernels(gpu, num_kv, kv_groups, max_blocks):
                                           one.data_ptr(), num_kv, kv_groups, max_blocks, 0.9, sphkv_lib.current_stream())
     assert rc == 0
     np.testing.assert_allclose(one.cpu().numpy(), want, rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("num_kv,kv_groups,max_blocks", [(2, 4, 64), (2, 4, 512), (2, 4, 513), (2, 8, 2048), (1, 9, 768)])
+def test_omega_ema_takes_a_workspace_of_the_queried_size(gpu, num_kv, kv_groups, max_blocks):
+    # 0 bytes among them: then the pointer is left alone
+    import sphkv_lib
+    lib, rng, nq = sphkv_lib.load(), np.random.default_rng(max_blocks), num_kv * kv_groups
+    m = (rng.standard_normal((nq, max_blocks)) * 5).astype(np.float32)
+    l = rng.random((nq, max_blocks)).astype(np.float32)
+    prev = rng.random((num_kv, max_blocks)).astype(np.float32)
+    ml, om = torch.from_numpy(np.stack([m, l], axis=-1)).to(gpu), _t(prev, gpu)
+    need = lib.sphkv_omega_ema_workspace_bytes(num_kv, kv_groups, max_blocks)
+    ws = torch.full((need // 4 + 2,), float("nan"), device=gpu)
+    assert lib.sphkv_omega_ema_ws(ml.data_ptr(), ml.data_ptr() + 4, ml.stride(0), 2, om.data_ptr(), om.data_ptr(), num_kv,
+                                  kv_groups, max_blocks, 0.9, ws.data_ptr(), need, sphkv_lib.current_stream()) == 0
+    assert torch.isnan(ws[need // 4:]).all()
+    np.testing.assert_allclose(om.cpu().numpy(), oracle.omega_ema(m, l, prev, num_kv, kv_groups, 0.9), rtol=1e-5, atol=1e-7)
