@@ -523,15 +523,17 @@ int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_
                     const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
                     int32_t max_blocks, float ema_beta, void* stream);
 /*
- * sphkv_omega_ema with device scratch for long tables: _workspace_bytes gives
- * what it wants (0: none, one kernel is as fast; negative on bad sizes), and
- * with that many bytes (8-byte aligned, contents irrelevant, free again when
- * the call has run) the pages are read by workgroups of 256 instead of one per
- * kv head.  workspace NULL, or a table that wants none (any workspace is taken
- * and left alone): as sphkv_omega_ema.  Calls that share a workspace must not
- * run concurrently.
+ * sphkv_omega_ema with device scratch for long tables: _workspace_wanted gives
+ * what it uses at these sizes and page stride (0: none, one kernel is as fast;
+ * negative on bad sizes), _workspace_bytes what is enough at any stride.  With
+ * that many bytes (8-byte aligned, contents irrelevant, free again when the
+ * call has run) the pages are read by workgroups of 256 instead of one per kv
+ * head.  workspace NULL, or a table that wants none (any workspace is taken and
+ * left alone): as sphkv_omega_ema.  Calls that share a workspace must not run
+ * concurrently.
  */
 int64_t sphkv_omega_ema_workspace_bytes(int32_t num_kv, int32_t kv_groups, int32_t max_blocks);
+int64_t sphkv_omega_ema_workspace_wanted(int32_t num_kv, int32_t kv_groups, int32_t max_blocks, int64_t page_stride);
 int sphkv_omega_ema_ws(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,
                        const float* omega_prev, float* omega_out, int32_t num_kv, int32_t kv_groups,
                        int32_t max_blocks, float ema_beta, void* workspace, int64_t workspace_bytes, void* stream);

@@ -884,8 +884,8 @@ static int omega_ema(const char* fn, const float* m_q, const float* l_q, int64_t
     return fail(SPHKV_EINVAL, "%s: kv_groups must be 1..%d", fn, sphkv::kOmegaMaxGroups);
   if (q_stride < 0 || page_stride < 0) return fail(SPHKV_EINVAL, "%s: negative stride", fn);
   if (num_kv == 0 || max_blocks == 0) return ok();
-  // (a short table runs in one kernel, whatever workspace is offered)
-  const bool split = ws && max_blocks > sphkv::kOmegaSplitBlocks &&
+  // (a table that wants one kernel gets it, whatever workspace is offered)
+  const bool split = ws && sphkv::omega_split(num_kv, kv_groups, max_blocks, page_stride) &&
                      (int64_t)num_kv * kv_groups * ((max_blocks + 255) / 256) < ((int64_t)1 << 31);
   if (split) {
     const int64_t need = 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
@@ -907,10 +907,14 @@ int sphkv_omega_ema(const float* m_q, const float* l_q, int64_t q_stride, int64_
 
 int64_t sphkv_omega_ema_workspace_bytes(int32_t num_kv, int32_t kv_groups, int32_t max_blocks) {
   if (num_kv < 0 || max_blocks < 0 || kv_groups < 1 || kv_groups > sphkv::kOmegaMaxGroups) return -1;
-  // one workgroup per kv head reads up to kOmegaSplitBlocks pages as fast as
-  // two kernels do
   if (max_blocks <= sphkv::kOmegaSplitBlocks) return 0;
   return 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
+}
+
+int64_t sphkv_omega_ema_workspace_wanted(int32_t num_kv, int32_t kv_groups, int32_t max_blocks, int64_t page_stride) {
+  const int64_t n = sphkv_omega_ema_workspace_bytes(num_kv, kv_groups, max_blocks);
+  if (page_stride < 0) return -1;
+  return n > 0 && !sphkv::omega_split(num_kv, kv_groups, max_blocks, page_stride) ? 0 : n;
 }
 
 int sphkv_omega_ema_ws(const float* m_q, const float* l_q, int64_t q_stride, int64_t page_stride,

@@ -120,10 +120,31 @@ struct OmegaLaunch {
   float* ws;                                                        // omega_workspace_floats() floats, or NULL: one kernel
 };
 constexpr int kOmegaChunk = 256;         // pages per workgroup of the two-kernel form
-constexpr int kOmegaSplitBlocks = 512;   // most pages of the one-kernel form when a workspace is offered
+constexpr int kOmegaSplitBlocks = 512;   // most pages of tables that are never split
+constexpr int kOmegaFastBlocks = 4096, kOmegaFastGroups = 8;   // limits of the one-kernel form that reads a pair once
 // (max, sum) of each (q head, chunk), then (m, l) of each (q head, page)
 inline int64_t omega_workspace_floats(int32_t num_kv, int32_t kv_groups, int32_t max_blocks) {
-  return 2 * (int64_t)num_kv * kv_groups * ((max_blocks + kOmegaChunk - 1) / kOmegaChunk + (int64_t)max_blocks);
+  return 2 * (int64_t)num_kv * kv_groups * (((int64_t)max_blocks + kOmegaChunk - 1) / kOmegaChunk + (int64_t)max_blocks);
+}
+// Does the two-kernel form pay for its second launch and scratch?  On the GPU
+// it is never slower (8 kv heads, dh 128, 513 / 2,048 / 4,096 blocks: 0.4 / 2.1
+// / 5.8 us sooner at 1 q head per kv head, 1.4 / 8.2 / 18.4 at 4, 5.1 / 17.4 /
+// 46.7 at 8), but they cost the caller's host 4 us, and a Mode-A step (append,
+// decode, this) is bound by the host up to about 36 us.  So it is taken where
+// the step's GPU work passes that: 24 us + 1.3 ns x (num_kv * pages * page
+// stride / 256 for the decode over pages of 16 tokens + a line of the vector
+// cache per pair here + 4,000 past 4 q heads, whose one-kernel form holds twice
+// the registers).  Per step, one kernel / two: 8 kv heads x 4 at dh 128 1,024
+// blocks 35.7 / 36.8 us, 1,536 40.4 / 37.0; x 1 1,536 34.2 / 34.3, 2,048 37.0 /
+// 35.0; x 8 384 36.4 / 37.2, 513 38.4 / 37.1; dh 64 x 4 1,536 34.4 / 37.8,
+// 2,048 38.5 / 37.3.
+inline bool omega_split(int32_t num_kv, int32_t kv_groups, int32_t max_blocks, int64_t page_stride) {
+  if (max_blocks <= kOmegaSplitBlocks) return false;
+  const int64_t pages = (int64_t)num_kv * max_blocks, lines = (int64_t)kv_groups * max_blocks;
+  // (the form that reads every pair three times is the slowest from 513 blocks on)
+  if (max_blocks > kOmegaFastBlocks || kv_groups > kOmegaFastGroups) return true;
+  const int64_t stride = page_stride < 32 ? page_stride : 32;            // 32 floats: a line each
+  return pages * (page_stride < 256 ? page_stride : 256) / 256 + lines * stride / 32 + (kv_groups > 4 ? 4000 : 0) >= 9400;
 }
 
 constexpr int kPoolBuildMaxG = 256;

@@ -1116,7 +1116,7 @@ namespace sphkv {
 // -- w = exp(max(m - max_p m, -60)) * l, mass = w / max(sum w, 1e-12) -- the
 // masses are averaged over each kv head's q heads and blended into omega:
 // omega' = omega * beta + mass * (1 - beta).  One workgroup per kv head, or
-// (a workspace, past kOmegaSplitBlocks blocks) one per 256 pages of a q head.
+// (a workspace and a long table, omega_split) one per 256 pages of a q head.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float block_reduce(float v, bool is_max, float* red) {
   for (int o = 32; o >= 1; o >>= 1) {
@@ -1337,7 +1337,7 @@ int launch_omega(const OmegaLaunch& L, hipStream_t stream) {
     else
       hipLaunchKernelGGL((omega_ema_fast_kernel<4, KG, 1024>), dim3(L.num_kv), dim3(1024), 0, stream, L, (int)adjacent);
   };
-  if (L.kv_groups <= 8 && L.max_blocks <= 4096) {
+  if (L.kv_groups <= kOmegaFastGroups && L.max_blocks <= kOmegaFastBlocks) {
     if (L.kv_groups <= 4) fast(std::integral_constant<int, 4>());
     else fast(std::integral_constant<int, 8>());
   } else {

@@ -6,7 +6,7 @@ Same argument meaning as the reference: m_q, l_q are the [num_q, max_blocks]
 (m, l) views of the decode's partial_scratch ([..., 0] and [..., 1]); the
 strided views are read in place.  Returns the new omega [num_kv, max_blocks]
 fp32 (out of place, like the reference; pass `out=omega_prev` to update in
-place).  One HIP kernel (two past 512 blocks); raises if libsphkv.so is missing.
+place).  One HIP kernel (two for long tables); raises if libsphkv.so is missing.
 """
 from __future__ import annotations
 
@@ -24,8 +24,8 @@ EMA_BETA = 0.9          # spherical_kv_pipeline.py EMA_BETA
 
 
 @lru_cache(maxsize=256)
-def _workspace_bytes(num_kv: int, kv_groups: int, max_blocks: int) -> int:
-    return _lib.sphkv_omega_ema_workspace_bytes(num_kv, kv_groups, max_blocks)
+def _workspace_bytes(num_kv: int, kv_groups: int, max_blocks: int, page_stride: int) -> int:
+    return _lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, max_blocks, page_stride)
 
 
 def _view_ok(t: torch.Tensor, name: str) -> None:
@@ -49,7 +49,7 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
         out = torch.empty_like(omega_prev)
     elif out.dtype != torch.float32 or not out.is_contiguous() or out.shape != omega_prev.shape:
         raise ValueError("out must be a contiguous fp32 tensor shaped like omega_prev")
-    need = _workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks))
+    need = _workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks), m_q.stride(1))
     if need <= 0:                                        # one kernel (and, for bad sizes, the call's own error)
         rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(),
                                   out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),

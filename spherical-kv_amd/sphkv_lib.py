@@ -69,6 +69,7 @@ SIGNATURES = {
                                         I32, F32, I32, P]),
     "sphkv_omega_ema": (ctypes.c_int, [P, P, I64, I64, P, P, I32, I32, I32, F32, P]),
     "sphkv_omega_ema_workspace_bytes": (I64, [I32, I32, I32]),
+    "sphkv_omega_ema_workspace_wanted": (I64, [I32, I32, I32, I64]),
     "sphkv_omega_ema_ws": (ctypes.c_int, [P, P, I64, I64, P, P, I32, I32, I32, F32, P, I64, P]),
     "sphkv_plan_pages_work_ints": (I64, [I32, I32, I32]),
     "sphkv_plan_pages_count": (ctypes.c_int, [P, I64, P, I32, I32, I32, I32, P, I64, P, P, P]),

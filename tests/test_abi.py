@@ -247,16 +247,36 @@ def test_omega_ema_workspace_query_and_call_agree():
     ws = ctypes.create_string_buffer(64)
     at = (ctypes.addressof(ws) + 7) & ~7
     for kv, g, n in ((8, 4, 1), (8, 4, 512), (8, 4, 513), (1, 8, 4096), (2, 9, 5000)):
-        need = lib.sphkv_omega_ema_workspace_bytes(kv, g, n)
+        need = lib.sphkv_omega_ema_workspace_wanted(kv, g, n, 130)
         assert need >= 0
         for size, msg in ((need, "null pointer"),) + (((need - 1, "workspace needs"),) if need else ()):
-            assert lib.sphkv_omega_ema_ws(None, None, 130, 2, None, None, kv, g, n, 0.9, at, size, None) == -1
+            assert lib.sphkv_omega_ema_ws(None, None, 130, 130, None, None, kv, g, n, 0.9, at, size, None) == -1
             assert msg in lib.sphkv_last_error().decode()
         if need:
-            assert lib.sphkv_omega_ema_ws(None, None, 130, 2, None, None, kv, g, n, 0.9, at + 4, need, None) == -1
+            assert lib.sphkv_omega_ema_ws(None, None, 130, 130, None, None, kv, g, n, 0.9, at + 4, need, None) == -1
             assert "8-byte aligned" in lib.sphkv_last_error().decode()
     assert lib.sphkv_omega_ema_workspace_bytes(8, 4, 512) == 0
     assert lib.sphkv_omega_ema_workspace_bytes(8, 0, 512) < 0 and lib.sphkv_omega_ema_workspace_bytes(-1, 4, 512) < 0
+
+
+@pytest.mark.parametrize("dh,num_kv,kv_groups,max_blocks,two", [
+    # steps bound by the host with one kernel, where a second launch costs 4 us
+    (128, 4, 4, 551, False), (128, 8, 1, 1024, False), (128, 8, 4, 1024, False), (64, 8, 4, 1536, False),
+    (64, 8, 8, 513, False), (128, 8, 8, 512, False), (128, 4, 4, 1024, False), (64, 4, 2, 3072, False),
+    # bound by the GPU
+    (128, 8, 1, 2048, True), (128, 8, 4, 1536, True), (128, 8, 4, 2048, True), (128, 8, 8, 513, True),
+    (64, 8, 4, 2048, True), (64, 8, 8, 1024, True), (128, 4, 4, 2048, True),
+    # only the three-pass kernel is left
+    (128, 1, 1, 4097, True), (64, 1, 9, 513, True), (64, 1, 9, 512, False),
+])
+def test_omega_ema_second_kernel_where_the_step_is_bound_by_the_gpu(dh, num_kv, kv_groups, max_blocks, two):
+    lib = sphkv_lib.load()
+    want = lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, max_blocks, dh + 2)
+    assert want == (lib.sphkv_omega_ema_workspace_bytes(num_kv, kv_groups, max_blocks) if two else 0)
+    assert lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, max_blocks, -1) < 0
+    # pairs that share lines want it no sooner, and a longer table no later
+    assert lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, max_blocks, 2) <= want
+    assert lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, 2 * max_blocks, dh + 2) >= want
 
 
 def test_noalloc_refuses_work_beyond_its_scratch():

@@ -273,3 +273,29 @@ def test_omega_ema_takes_a_workspace_of_the_queried_size(gpu, num_kv, kv_groups,
                                   kv_groups, max_blocks, 0.9, ws.data_ptr(), need, sphkv_lib.current_stream()) == 0
     assert torch.isnan(ws[need // 4:]).all()
     np.testing.assert_allclose(om.cpu().numpy(), oracle.omega_ema(m, l, prev, num_kv, kv_groups, 0.9), rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("num_kv,kv_groups,max_blocks,dh", [
+    (8, 8, 513, 128), (8, 8, 1025, 64), (8, 4, 1536, 128), (8, 4, 2048, 64), (8, 1, 2049, 128), (3, 2, 4096, 128)])
+def test_omega_ema_of_strided_pairs(gpu, num_kv, kv_groups, max_blocks, dh):
+    # (m, l) a whole partial apart, as the decode leaves them, at sizes that
+    # take two kernels (a last chunk of one page, whole ones, more than one
+    # chunk, a chunk and a head without valid pages) and through one kernel
+    import omega_ema
+    import sphkv_lib
+    lib, rng, nq = sphkv_lib.load(), np.random.default_rng(max_blocks + dh), num_kv * kv_groups
+    assert lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, max_blocks, dh + 2) > 0
+    m = (rng.standard_normal((nq, max_blocks)) * 20).astype(np.float32)
+    l = np.where(rng.random((nq, max_blocks)) < 0.8, rng.random((nq, max_blocks)) * 3, 0.0).astype(np.float32)
+    l[:, 256:512] = 0.0
+    l[-1] = 0.0
+    prev = rng.random((num_kv, max_blocks)).astype(np.float32)
+    part = torch.full((nq, max_blocks, dh + 2), float("nan"), device=gpu)
+    part[:, :, 0], part[:, :, 1] = _t(m, gpu), _t(l, gpu)
+    want = oracle.omega_ema(m, l, prev, num_kv, kv_groups, 0.9)
+    got = omega_ema.omega_ema(part[..., 0], part[..., 1], _t(prev, gpu), num_kv, kv_groups, max_blocks, 0.9)
+    np.testing.assert_allclose(got.cpu().numpy(), want, rtol=1e-5, atol=1e-7)
+    one = _t(prev, gpu)
+    assert lib.sphkv_omega_ema(part.data_ptr(), part.data_ptr() + 4, part.stride(0), dh + 2, one.data_ptr(), one.data_ptr(),
+                               num_kv, kv_groups, max_blocks, 0.9, sphkv_lib.current_stream()) == 0
+    np.testing.assert_allclose(one.cpu().numpy(), want, rtol=1e-5, atol=1e-7)
