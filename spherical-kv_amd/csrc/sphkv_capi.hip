@@ -885,8 +885,7 @@ static int omega_ema(const char* fn, const float* m_q, const float* l_q, int64_t
   if (q_stride < 0 || page_stride < 0) return fail(SPHKV_EINVAL, "%s: negative stride", fn);
   if (num_kv == 0 || max_blocks == 0) return ok();
   // (a table that wants one kernel gets it, whatever workspace is offered)
-  const bool split = ws && sphkv::omega_split(num_kv, kv_groups, max_blocks, page_stride) &&
-                     (int64_t)num_kv * kv_groups * ((max_blocks + 255) / 256) < ((int64_t)1 << 31);
+  const bool split = ws && sphkv::omega_split(num_kv, kv_groups, max_blocks, page_stride);
   if (split) {
     const int64_t need = 4 * sphkv::omega_workspace_floats(num_kv, kv_groups, max_blocks);
     if (ws_bytes < need || ((uintptr_t)ws & 7) != 0)

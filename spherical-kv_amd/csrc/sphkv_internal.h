@@ -141,6 +141,9 @@ inline int64_t omega_workspace_floats(int32_t num_kv, int32_t kv_groups, int32_t
 inline bool omega_split(int32_t num_kv, int32_t kv_groups, int32_t max_blocks, int64_t page_stride) {
   if (max_blocks <= kOmegaSplitBlocks) return false;
   const int64_t pages = (int64_t)num_kv * max_blocks, lines = (int64_t)kv_groups * max_blocks;
+  // (a grid holds fewer than 2^32 threads: one per pair, whole workgroups)
+  if ((int64_t)num_kv * kv_groups * (((int64_t)max_blocks + kOmegaChunk - 1) / kOmegaChunk) >= ((int64_t)1 << 32) / kOmegaChunk)
+    return false;
   // (the form that reads every pair three times is the slowest from 513 blocks on)
   if (max_blocks > kOmegaFastBlocks || kv_groups > kOmegaFastGroups) return true;
   const int64_t stride = page_stride < 32 ? page_stride : 32;            // 32 floats: a line each

@@ -279,6 +279,15 @@ def test_omega_ema_second_kernel_where_the_step_is_bound_by_the_gpu(dh, num_kv, 
     assert lib.sphkv_omega_ema_workspace_wanted(num_kv, kv_groups, 2 * max_blocks, dh + 2) >= want
 
 
+def test_omega_ema_second_kernel_within_a_grid():
+    # the two-kernel form launches a thread per pair, and a grid holds fewer
+    # than 2^32 of them: larger tables keep one kernel
+    lib = sphkv_lib.load()
+    for kv, g, n in ((1 << 18, 8, 2048), (1 << 16, 16, 4096), (1 << 12, 128, 8192), (1, 1, 2 ** 31 - 1)):
+        fits = kv * g * -(-n // 256) * 256 < 1 << 32
+        assert (lib.sphkv_omega_ema_workspace_wanted(kv, g, n, 130) > 0) == fits, (kv, g, n)
+
+
 def test_noalloc_refuses_work_beyond_its_scratch():
     # the size check runs before any device access
     lib = sphkv_lib.load()
