@@ -519,7 +519,10 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
 #pragma unroll
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, D[b][i]);
       }
-    const float thr = rows_max(mx) - (kGapSlack * unit + 1e-30f);
+    // (an infinite key's products are infinite or NaN and rank nothing: no
+    // candidates, every code scored)
+    float thr = rows_max(mx) - (kGapSlack * unit + 1e-30f);
+    thr = thr > 0.1f * kNoSim ? thr : __builtin_nanf("");
     uint32_t lo = 0u, hi = 0u;
 #pragma unroll
     for (int b = 0; b < 4; ++b)

@@ -233,3 +233,35 @@ def test_encode_small_gaps_scales_and_bit_patterns(gpu, dh, H, L, fp32):
     assert (r[comp].view(np.uint32) == cpu["r"][comp].view(np.uint32)).all()
     assert (pool.pages.cpu().numpy() == cpu["pages"]).all()
     assert (pool.v_pool.cpu().numpy().view(np.uint16) == cpu["v_pool"].view(np.uint16)).all()
+
+
+def _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh):
+    plan = fmt.plan_pages(tier_of, None, 1, H, dh, 16, rng=rng)
+    wl = synth.Workload(name="codes", dh=dh, num_kv=H, gqa=1, num_seqs=1, lengths=[L], rope_theta=5e5, codebooks=cbs,
+                        K=[K], V=[np.zeros((H, L, dh), np.float16)], q=np.zeros((1, H, dh), np.float16),
+                        tier_of=tier_of, plan=plan)
+    pool, r_out, c_out = ops.build_pool_gpu(wl, gpu, with_codes=True)
+    torch.cuda.synchronize()
+    with np.errstate(all="ignore"):
+        cpu = oracle.build_pool(wl, with_codes=True)
+    return r_out.cpu().numpy(), c_out.cpu().numpy(), cpu
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_encode_infinite_keys_take_the_first_code(gpu, fp32):
+    # a group with infinities has NaN directions and NaN similarities: the
+    # first code wins, however the unnormalised products rank (several
+    # infinities leave some of them -inf and the rest NaN)
+    rng = np.random.default_rng(5)
+    H, L, dh = 2, 400, 128
+    tier_of = [rng.choice(np.array([1, 2, 3], np.int32), size=L) for _ in range(H)]
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    K = rng.standard_normal((H, L, dh)).astype(np.float32 if fp32 else np.float16)
+    for h in range(H):
+        for t in range(L):
+            for j in range(0, dh, 16):
+                n = int(rng.integers(0, 7))
+                K[h, t, j + rng.choice(16, n, replace=False)] = np.inf * rng.choice([-1, 1], n)
+    log(f"infinite keys fp32={fp32}")
+    _, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
+    assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
