@@ -86,14 +86,16 @@ struct EncodeLds {
 // Gap between the two largest approximate similarities S = <x, c> (in units of
 // r = |x|) past which the largest is the exact first maximum.  |S - s r| <=
 // eps r for the exactly scored s, from: the codebook row's two fp16 terms
-// (2^-20), fp32 keys' two terms (2^-19), the fp32 sums of up to 96 products
-// (6e-6), the six low bits of S that carry the code (4e-6), the rounding of
-// the exact chain and of its direction (2.5e-6); eps < 1.6e-5 for rows with
-// |c|^2 <= 1.1.  The unit keeps fp16 denormals.  At 4e-5 about 0.06 % of the
-// token-groups of Gaussian keys are scored exactly; fp16 terms of the
-// direction alone need 5e-3, which left more than one candidate to one lane
-// of nearly every wave.
-constexpr float kGapSlack = 4e-5f;
+// (2^-20, and 2^-24 sqrt(g) where the second is denormal: the unit keeps fp16
+// denormals), fp32 keys' two terms (2^-19), the fp32 sums of up to 96 products
+// (5.7e-6), the six low bits of S that carry the code (63 ulp: 7.5e-6 at the
+// bottom of a binade), the rounding of the exact chain and of its direction
+// (2e-6).  With rows of |c|^2 <= 1.1 that is eps < 1.95e-5, and two values may
+// err apart: 3.9e-5, which the slack passes by a quarter.  About 0.05 % of the
+// token-groups of Gaussian keys are scored exactly; fp16 terms of the direction
+// alone need 5e-3, which left more than one candidate to one lane of nearly
+// every wave.
+constexpr float kGapSlack = 5e-5f;
 // The bound above scales with |c|: it holds for rows with |c|^2 within
 // kUnitTol of 1.  Against a codebook with any other row (scaled or
 // unnormalised rows: _encode_keys_with_codebooks accepts any codebook, only
