@@ -101,6 +101,10 @@ constexpr float kGapSlack = 5e-5f;
 // unnormalised rows: _encode_keys_with_codebooks accepts any codebook, only
 // codebook_loader.py:43-44 normalises) every code is scored exactly.
 constexpr float kUnitTol = 0.1f;
+// fp32 keys are ranked at length 256, through their norm.  Below 1e-18 the
+// squares lose bits to underflow and the norm with them (at 4e-23 it is 3 times
+// too short), so such groups are scored exactly.
+constexpr float kMinNorm = 1e-18f;
 constexpr int kOpenCode = 0x100;       // a code left to the exact scoring
 constexpr float kNoSim = -1e30f;       // no similarity yet (finite: its low bits carry a code too)
 
@@ -482,8 +486,8 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
   // first code wins (8,192 x 8 tokens at three tiers, every key zero: 69 -> 21
   // us; every eighth: 70 -> 26; none: 26.7 -> 26.8)
   const bool zero = !K32 && r == 0.f;
-  const bool open = live && (((bad_pages >> j) & 1u) ||
-                             (!zero && (!(a0 - c0 > kGapSlack * unit + 1e-30f) || !(a0 > 0.1f * kNoSim))));
+  const bool open = live && (((bad_pages >> j) & 1u) || (!zero && (!(a0 - c0 > kGapSlack * unit + 1e-30f) ||
+                                                                   !(a0 > 0.1f * kNoSim) || (K32 && r < kMinNorm))));
   code = live ? (open ? kOpenCode : zero ? 0 : code) : 0;
 }
 
@@ -536,7 +540,8 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
     hi = rows_or(hi << (4 * j));
     const uint64_t mk = (uint64_t)lo | ((uint64_t)hi << 32);
     const bool naive = mt.ord * 16 * C < 400;
-    if (open && j == jj && mk != 0 && __builtin_popcountll(mk) <= 8 && (naive || mt.ord > 1)) {
+    if (open && j == jj && mk != 0 && __builtin_popcountll(mk) <= 8 && (naive || mt.ord > 1) &&
+        (!K32 || r >= kMinNorm)) {
       KeyRegs<16, K32> k;
       load_keys<16, K32>(a, mt.row * DH + 16 * w, true, nullptr, k);
       auto quad = [&](int q, float (&x)[4]) __attribute__((always_inline)) {
@@ -550,7 +555,7 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
       open = false;
     }
   }
-  // many ties (r = 0 among them), NaNs, non-unit rows and tier 3: every code
+  // many ties, NaNs, fp32 keys too small to rank, non-unit rows and tier 3: every code
   // scored, with the codebook rows as scalar operands, lanes of one (tier,
   // head) at a time
   uint64_t todo = __builtin_amdgcn_ballot_w64(open);

@@ -101,3 +101,23 @@ def test_ranking_stands_past_the_slack(g, C, fp32):
         kept += int(clear.sum())
         assert (top.argmax(1) == s.argmax(1))[clear].all()
     assert kept > 1000 and 2 * worst <= slack
+
+
+@pytest.mark.parametrize("g", [16, 32])
+def test_ranked_fp32_keys_have_the_length_that_the_slack_is_taken_in(g):
+    # the fp32 norm in the kernel's order (8 chains of fused multiply-adds, a
+    # float64 product and sum rounded once), from keys whose squares underflow
+    rng, least = np.random.default_rng(g), _constant("kMinNorm")
+    x = rng.standard_normal((20000, g))
+    x = (x / np.linalg.norm(x, axis=1, keepdims=True) * 10.0 ** rng.uniform(-23.5, -15, (20000, 1))).astype(F)
+    acc = np.zeros((len(x), 8), F)
+    for d in range(0, g, 8):
+        acc = (x[:, d:d + 8].astype(np.float64) ** 2 + acc).astype(F)
+    s = acc[:, 0]
+    for lane in range(1, 8):
+        s = s + acc[:, lane]
+    r, true = np.sqrt(s), np.linalg.norm(x.astype(np.float64), axis=1)
+    ranked = (r > 0) & (r >= F(least))
+    off = np.abs(true[ranked] / r[ranked] - 1)
+    assert ranked.sum() > 1000 and off.max() < 1e-6
+    assert np.abs(true[r > 0] / r[r > 0] - 1).max() > 0.5          # what the limit keeps out

@@ -265,3 +265,26 @@ def test_encode_infinite_keys_take_the_first_code(gpu, fp32):
     log(f"infinite keys fp32={fp32}")
     _, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
     assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
+
+
+def test_encode_tiny_fp32_keys(gpu):
+    # norms from where their squares are denormal (so that the fp32 norm is off
+    # by up to a factor) to ordinary ones, gaps between the two best centroids
+    # of 1e-6 to 1e-3
+    rng = np.random.default_rng(6)
+    H, L, dh = 2, 1500, 128
+    tier_of = [rng.choice(np.array([1, 2, 3], np.int32), size=L) for _ in range(H)]
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    K = np.zeros((H, L, dh), np.float32)
+    for h in range(H):
+        for t in range(L):
+            cb = cbs[int(tier_of[h][t])][h]
+            G, C, g = cb.shape
+            for j in range(G):
+                a, b = rng.choice(C, size=2, replace=False)
+                v = cb[j, a] + cb[j, b] * np.float32(1 - 10.0 ** rng.uniform(-6, -3))
+                K[h, t, j * g:(j + 1) * g] = v * np.float32(10.0 ** rng.uniform(-23.2, -17 if t % 2 else -22))
+    log("tiny fp32 keys")
+    r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
+    assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
+    assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
