@@ -398,9 +398,17 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
   constexpr int RB = 2 * GG;                             // bytes per staged row
   const int j = lane >> 4, t = lane & 15;
   r = 0.f;
+  bool zero = false;                                     // every value of a live group is zero
   uint8_t* dst = xs + PB * j + RB * t;
   if constexpr (K32) {
     if (live) r = torch_norm(k.f, GG);
+    const bool none = live && r == 0.f;                  // (also where every square underflows)
+    if (__builtin_amdgcn_ballot_w64(none)) {
+      uint32_t any = 0u;
+#pragma unroll
+      for (int i = 0; i < GG; ++i) any |= __builtin_bit_cast(uint32_t, k.f[i]) << 1;
+      zero = none && any == 0u;
+    }
     // scaled to length 256 (a factor common to a token's similarities leaves
     // their order): high and low fp16 halves
     const float sc = 256.f * __builtin_amdgcn_rcpf(r);
@@ -423,6 +431,7 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
 #pragma unroll
     for (int i = 0; i < GG; ++i) x[i] = (float)k.h[i / 8][i % 8];
     if (live) r = torch_norm(x, GG);
+    zero = live && r == 0.f;
   }
   wave_lds_sync();
   float m1[kSetPages], m2[kSetPages];
@@ -482,10 +491,9 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
   top2_merge(a0, c0, b0, d0);
   code = (int)(__builtin_bit_cast(uint32_t, a0) & 63u);
   const float unit = K32 ? 256.f : r;
-  // a zero fp16 key (r is 0 for no other) scores 0 on every finite row: the
-  // first code wins (8,192 x 8 tokens at three tiers, every key zero: 69 -> 21
-  // us; every eighth: 70 -> 26; none: 26.7 -> 26.8)
-  const bool zero = !K32 && r == 0.f;
+  // a zero key scores 0 on every finite row: the first code wins (8,192 x 8
+  // tokens at three tiers, every fp16 key zero: 69 -> 21 us; every eighth: 70
+  // -> 27; fp32: 92 -> 33 and 91 -> 41; none: 28 and 42)
   const bool open = live && (((bad_pages >> j) & 1u) || (!zero && (!(a0 - c0 > kGapSlack * unit + 1e-30f) ||
                                                                    !(a0 > 0.1f * kNoSim) || (K32 && r < kMinNorm))));
   code = live ? (open ? kOpenCode : zero ? 0 : code) : 0;
