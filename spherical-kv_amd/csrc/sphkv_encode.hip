@@ -204,35 +204,59 @@ __device__ __forceinline__ void encode_group(const EncodeArgs& a, int64_t kofs, 
 }
 
 // The code of one token's 16-value group among the candidate codes of mask mk
-// (their rows at cb + 16 c), scored exactly in ascending order (calls over one
-// token at C = 64, whose order is code_sim_m1's, are left to encode_group).
-// quad(q) gives values 4 q .. 4 q + 3 of the group; four at a time, so that
-// the kernel's register count is not set here.
-template <bool K32, typename Q>
-__device__ __forceinline__ int score_candidates(Q quad, float r, bool naive, const float* cb, uint64_t mk) {
-  const float den = __fadd_rn(r, 1e-8f);
+// (not empty; their rows at cb + 16 c), scored exactly in ascending order
+// (calls over one token at C = 64, whose order is code_sim_m1's, are left to
+// encode_group).  Rows are loaded two at a time: a tie is most often of two.
+__device__ __forceinline__ int score_candidates(const float* dir, bool naive, const float* cb, uint64_t mk) {
   float best_sim = 0.f;
   int best = -1;
   while (mk) {
-    const int c = (int)__builtin_ctzll(mk);
-    mk &= mk - 1;
-    float4 w[4];
+    int c[2];
+    float4 w[2][4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) w[q] = *reinterpret_cast<const float4*>(cb + 16 * c + 4 * q);
-    float sc = 0.f;
+    for (int i = 0; i < 2; ++i) {
+      c[i] = i && !mk ? c[0] : (int)__builtin_ctzll(mk);
+      mk &= mk - 1;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      float x[4], d[4];
-      quad(q, x);
-      group_directions<4>(x, den, !K32, d);
-      const float v[4] = {w[q].x, w[q].y, w[q].z, w[q].w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) sc = naive ? __fadd_rn(sc, __fmul_rn(d[e], v[e])) : __builtin_fmaf(d[e], v[e], sc);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int q = 0; q < 4; ++q) w[i][q] = *reinterpret_cast<const float4*>(cb + 16 * c[i] + 4 * q);
     }
-    if (best < 0 || sc > best_sim) { best_sim = sc; best = c; }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      float sc = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float v[4] = {w[i][q].x, w[i][q].y, w[i][q].z, w[i][q].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          sc = naive ? __fadd_rn(sc, __fmul_rn(dir[4 * q + e], v[e])) : __builtin_fmaf(dir[4 * q + e], v[e], sc);
+      }
+      if (best < 0 || sc > best_sim) { best_sim = sc; best = c[i]; }
+    }
   }
   return best;
+}
+
+// Mask mk (not empty) without the codes whose row repeats its first one's: they
+// score the same, and the first wins.
+__device__ __forceinline__ uint64_t drop_repeats(const float* cb, uint64_t mk) {
+  const uint4* first = reinterpret_cast<const uint4*>(cb + 16 * (int)__builtin_ctzll(mk));
+  uint4 f[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) f[q] = first[q];
+  uint64_t rest = mk & (mk - 1);
+  while (rest) {
+    const int c = (int)__builtin_ctzll(rest);
+    rest &= rest - 1;
+    const uint4* row = reinterpret_cast<const uint4*>(cb + 16 * c);
+    uint32_t d = 0u;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint4 v = row[q];
+      d |= (v.x ^ f[q].x) | (v.y ^ f[q].y) | (v.z ^ f[q].z) | (v.w ^ f[q].w);
+    }
+    if (d == 0u) mk &= ~(1ull << c);
+  }
+  return mk;
 }
 
 // hi + lo = x to 2^-20 |x|, as fp16 (both terms rounded towards zero).
@@ -366,19 +390,17 @@ __device__ __forceinline__ floatx4 sims16(const Codebook& cb, int b, half4 B, ha
   return D;
 }
 
-// What the exact scoring needs of a token, loaded again where it runs (so that
-// the usual path holds none of it in registers).
+// What the second group size and the exact scoring need of a token, loaded
+// again where they run (so that the usual path does not hold it in registers).
 struct TokenMeta {
   int64_t row;
-  int tid, head, ord;
+  int ord;
 };
 template <bool CODES>
 __device__ __forceinline__ TokenMeta reload_token(const EncodeArgs& a, int pc, int t) {
   asm volatile("" : "+v"(pc));
   TokenMeta m;
   m.row = a.src_rows[(int64_t)pc * kTile + t];
-  m.tid = a.tier[pc];
-  m.head = max(a.seq_head[pc], 0) % a.num_kv;
   // the summation order follows torch's call over ord tokens: the page's own
   // count, or the caller's N (a whole head's tokens in one call)
   m.ord = CODES && a.order_n ? max(a.order_n[pc], 1) : min(max(a.count[pc], 0), kTile);
@@ -500,24 +522,30 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
 }
 
 // The wave's (token, group)s that encode_tokens left open, scored exactly.
-// Everything is loaded again, so that the usual path holds nothing for it.
+// Their metadata and fp32 keys are loaded again, so that the usual path holds
+// nothing for it.
 template <int DH, bool K32, bool CODES>
-__device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* xs, int PB, int pc, int w, int lane,
-                                           bool open, float& r, int& code) {
+__device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* xs, int PB, int pc, int tid_l, int head_l, int w, int lane,
+                                           bool open, Codebook& cb, float& r, int& code) {
   asm volatile("" : "+v"(lane));
   const int j = lane >> 4, t = lane & 15;
   const TokenMeta mt = reload_token<CODES>(a, pc, t);
   // a gap within the slack: the page's similarities again, for the codes
-  // within it, which are then scored exactly.  (A wave in 30 comes here; a
-  // scan of all 64 codes instead held up its workgroup by 2 to 3 us.)
+  // within it; then all pages' tokens together, codes of repeated rows without
+  // scoring.  A wave in 30 comes here for Gaussian keys and random rows, nearly
+  // every one against repeated rows, and what that costs is its round trips:
+  // scored page by page, with metadata and codebook loaded again for each,
+  // 8,192 x 8 fp16 tokens at three tiers took 64 us with one row of each group
+  // twice and 93 with every row, now 36 and 41 (fp32 keys 74 -> 55, 96 -> 63;
+  // without ties 27 and 42).  (Tier 3 by candidates too: 40 and 48.)
+  uint64_t mk = 0;                                       // this lane's token: codes within the slack
 #pragma unroll 1
   for (int jj = 0; jj < kSetPages; ++jj) {
-    const int tid = uniform(__builtin_amdgcn_readlane(mt.tid, 16 * jj));
+    const int tid = uniform(__builtin_amdgcn_readlane(tid_l, 16 * jj));
     if (((__builtin_amdgcn_ballot_w64(open) >> (16 * jj)) & 0xFFFFull) == 0 || tid == 3) continue;
-    const int h = uniform(__builtin_amdgcn_readlane(mt.head, 16 * jj));
+    const int h = uniform(__builtin_amdgcn_readlane(head_l, 16 * jj));
     const int C = tier_C(tid);
-    Codebook cb;
-    load_codebook<DH, false>(a, tid, h, w, lane, cb);
+    if (tid != cb.tid || h != cb.h) load_codebook<DH, false>(a, tid, h, w, lane, cb);
     if (cb.bad) continue;
     const uint8_t* xp = xs + PB * jj + 32 * t;
     const half4 B = *reinterpret_cast<const half4*>(xp + 8 * j);
@@ -546,20 +574,34 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
       }
     lo = rows_or(lo << (4 * j));
     hi = rows_or(hi << (4 * j));
-    const uint64_t mk = (uint64_t)lo | ((uint64_t)hi << 32);
+    if (j == jj) mk = (uint64_t)lo | ((uint64_t)hi << 32);
+  }
+  {
+    const int C = tid_l == 1 ? 64 : 16;
     const bool naive = mt.ord * 16 * C < 400;
-    if (open && j == jj && mk != 0 && __builtin_popcountll(mk) <= 8 && (naive || mt.ord > 1) &&
-        (!K32 || r >= kMinNorm)) {
-      KeyRegs<16, K32> k;
-      load_keys<16, K32>(a, mt.row * DH + 16 * w, true, nullptr, k);
-      auto quad = [&](int q, float (&x)[4]) __attribute__((always_inline)) {
+    const float* rows = (tid_l == 1 ? a.cb[1] : a.cb[2]) + ((int64_t)head_l * (DH / 16) + w) * C * 16;
+    bool few = open && mk != 0 && __builtin_popcountll(mk) <= 8 && (naive || mt.ord > 1) && (!K32 || r >= kMinNorm);
+    if (few) {
+      mk = drop_repeats(rows, mk);
+      if ((mk & (mk - 1)) == 0) {
+        code = (int)__builtin_ctzll(mk);
+        few = open = false;
+      }
+    }
+    if (few) {
+      float x[16], dir[16];
+      if constexpr (K32) {
+        KeyRegs<16, K32> k;
+        load_keys<16, K32>(a, mt.row * DH + 16 * w, true, nullptr, k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          if constexpr (K32) x[e] = k.f[4 * q + e];
-          else x[e] = (float)k.h[q / 2][4 * (q & 1) + e];
-        }
-      };
-      code = score_candidates<K32>(quad, r, naive, a.cb[tid] + ((int64_t)h * (DH / 16) + w) * C * 16, mk);
+        for (int i = 0; i < 16; ++i) x[i] = k.f[i];
+      } else {
+        const half8* src = reinterpret_cast<const half8*>(xs + PB * j + 32 * t);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = (float)src[i / 8][i % 8];
+      }
+      group_directions<16>(x, __fadd_rn(r, 1e-8f), !K32, dir);
+      code = score_candidates(dir, naive, rows, mk);
       open = false;
     }
   }
@@ -569,9 +611,9 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
   uint64_t todo = __builtin_amdgcn_ballot_w64(open);
   while (todo) {
     const int lead = (int)__builtin_ctzll(todo);                 // first lane not yet encoded
-    const int tid = uniform(__builtin_amdgcn_readlane(mt.tid, lead));
-    const int h = uniform(__builtin_amdgcn_readlane(mt.head, lead));
-    const bool mine = open && mt.tid == tid && mt.head == h;
+    const int tid = uniform(__builtin_amdgcn_readlane(tid_l, lead));
+    const int h = uniform(__builtin_amdgcn_readlane(head_l, lead));
+    const bool mine = open && tid_l == tid && head_l == h;
     todo &= ~__builtin_amdgcn_ballot_w64(mine);
     const int g = uniform(tier_g(tid)), C = uniform(tier_C(tid));
     const uint64_t cba = (uint64_t)(a.cb[tid] + ((int64_t)h * (DH / g) + w) * C * g);
@@ -738,7 +780,7 @@ __global__ __launch_bounds__(kEncWaves * 64) __attribute__((amdgpu_waves_per_eu(
     const bool open = (((comp16 | comp32) >> lane) & 1ull) && code == kOpenCode;
     if (__builtin_amdgcn_ballot_w64(open)) {
       float r = sm.r[64 * set + lane][w];
-      score_open<DH, K32, CODES>(a, xs, PB, pc, w, lane, open, r, code);
+      score_open<DH, K32, CODES>(a, xs, PB, pc, tid_l, head_l, w, lane, open, cb, r, code);
       if (open) {
         sm.r[64 * set + lane][w] = r;
         sm.code[64 * set + lane][w] = code;

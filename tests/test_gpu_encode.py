@@ -288,3 +288,35 @@ def test_encode_tiny_fp32_keys(gpu):
     r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
     assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
     assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("kind", ["one", "twice", "four", "last_value", "zero_sign"])
+def test_encode_repeated_codebook_rows(gpu, kind, fp32):
+    # ties of whole rows go to the first code; rows that differ in their last
+    # value or in a zero's sign are scored like any others; pages of 1 token
+    # (torch's M = 1 order) to 16, of every tier
+    rng = np.random.default_rng(11)
+    H, L, dh = 2, 260, 128
+    lens = rng.permutation(np.r_[1, 2, 3, 17, 33])
+    tier_of = [np.concatenate([np.full(lens[0], 1), rng.integers(1, 4, L - lens[0])]).astype(np.int32) for _ in range(H)]
+    tier_of[1][:] = np.where(np.arange(L) == 7, 1, np.where(np.arange(L) < 200, 2, 3))         # one token of tier 1
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    for tid, cb in cbs.items():
+        C = cb.shape[2]
+        if kind == "one":
+            cb[:, :, C - 1] = cb[:, :, 0]
+        elif kind == "four":
+            cb[:, :, C // 4:] = np.tile(cb[:, :, :C // 4], (1, 1, 3, 1))
+        else:
+            cb[:, :, C // 2:] = cb[:, :, :C // 2]
+        if kind == "last_value":
+            cb[:, :, C // 2:, -1] = np.nextafter(cb[:, :, C // 2:, -1], np.float32(2))
+        if kind == "zero_sign":
+            cb[:, :, :, 3] = 0
+            cb[:, :, C // 2:, 3] = -0.0
+    K = rng.standard_normal((H, L, dh)).astype(np.float32 if fp32 else np.float16)
+    log(f"repeated rows {kind} fp32={fp32}")
+    r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
+    assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
+    assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
