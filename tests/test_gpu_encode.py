@@ -320,3 +320,31 @@ def test_encode_repeated_codebook_rows(gpu, kind, fp32):
     r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
     assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
     assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+def test_encode_ties_of_negative_and_zero_similarities(gpu, fp32):
+    # every row in one half space and repeated, keys on its other side or
+    # orthogonal to all rows: the ranking's threshold lies below zero
+    rng = np.random.default_rng(17)
+    H, L, dh = 2, 300, 128
+    tier_of = [rng.integers(1, 4, L).astype(np.int32) for _ in range(H)]
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    K = np.zeros((H, L, dh))
+    for tid, cb in cbs.items():
+        G, C, g = cb.shape[1:]
+        rows = 0.3 * rng.standard_normal((H, G, C, g)) + 1
+        rows[..., g // 2:] = 0
+        rows /= np.linalg.norm(rows, axis=-1, keepdims=True)
+        cb[:] = rows
+        cb[:, :, C // 2:] = cb[:, :, :C // 2]
+        for h in range(H):
+            for t in np.flatnonzero(tier_of[h] == tid):
+                x = 0.2 * rng.standard_normal((G, g)) - 1
+                x[:, :g // 2] *= t % 5 > 0
+                K[h, t] = (x * 10.0 ** rng.uniform(-3, 2)).reshape(-1)
+    K = K.astype(np.float32 if fp32 else np.float16)
+    log(f"negative and zero similarities fp32={fp32}")
+    r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
+    assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
+    assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
