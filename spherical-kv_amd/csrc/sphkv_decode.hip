@@ -1161,7 +1161,7 @@ struct TailArgs {
 };
 
 constexpr int kTailThreads = 256;
-constexpr int kTailNarrowMax = 512;      // most workgroups of the narrow form (two per CU)
+constexpr int kTailNarrowMax = 512;      // most workgroups of the narrow form: two for each of the GPU's 256 CUs
 
 // Output floats of one tail workgroup: 128, or (wide) up to 512.  Each
 // workgroup of a (seq, head) repeats its loads, the new token's encode and the
@@ -1174,10 +1174,10 @@ __host__ __device__ constexpr int tail_slice(int dh, int gqa, bool wide) {
   return n < most ? n : most;
 }
 
-template <int DH, int GQA, bool WIDE>
+// SL: output floats of one workgroup (a slice), tail_slice.
+template <int DH, int GQA, int SL>
 __global__ __launch_bounds__(kTailThreads) void decode_tail_kernel(DecodeArgs a, TailArgs t) {
   constexpr int G3 = DH / 32, NJ = DH / 2, NS = kTailSlots;
-  constexpr int SL = tail_slice(DH, GQA, WIDE);        // output floats of one workgroup (a slice)
   constexpr int NSL = (GQA * DH) / SL;                 // slices per (seq, head)
   constexpr int HPS = SL / DH;                         // q heads per slice
   constexpr int COLS = SL / 4;                         // float4 columns of a slice
@@ -1651,11 +1651,12 @@ static int launch_decode_tail_t(const DecodeLaunch& L, const TailLaunch& T, hipS
   if ((T.mode & kTailDecode) && L.num_items > 0)
     launch_timed(decode_kernel<DH, GQA>, dim3(L.num_items), dim3(kDecodeWaves * 64), stream, L.work,
                  L.num_items, a);
-  constexpr int NSL = (GQA * DH) / tail_slice(DH, GQA, false), NSW = (GQA * DH) / tail_slice(DH, GQA, true);
-  if (nsh * NSL > kTailNarrowMax)
-    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, true>), dim3(nsh * NSW), dim3(kTailThreads), 0, stream, a, t);
+  // (up to 128 output floats both forms are the one kernel)
+  constexpr int SN = tail_slice(DH, GQA, false), SW = tail_slice(DH, GQA, true), NSN = GQA * DH / SN, NSW = GQA * DH / SW;
+  if (nsh * NSN > kTailNarrowMax)
+    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, SW>), dim3(nsh * NSW), dim3(kTailThreads), 0, stream, a, t);
   else if (nsh > 0)
-    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, false>), dim3(nsh * NSL), dim3(kTailThreads), 0, stream, a, t);
+    hipLaunchKernelGGL((decode_tail_kernel<DH, GQA, SN>), dim3(nsh * NSN), dim3(kTailThreads), 0, stream, a, t);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
