@@ -110,6 +110,14 @@ constexpr float kMinNorm = 1e-18f;
 // A code left to the exact scoring is the bits of its best approximate
 // similarity, at least this (values that small rank as zeros).
 constexpr uint32_t kOpenCode = 0x100;
+// Most codes of a wave that are scored one at a time.  Gaussian keys leave one
+// to a wave in 30, and such a wave ends its workgroup: the pass over pages and
+// candidates takes 5,000 cycles for one code as for 64, score_alone a fifth of
+// that.  8,192 x 8 tokens at three tiers 25.3 -> 22.4 us (fp32 keys 36.3 ->
+// 32.6), 4 x 500 of dh 64 6.7 -> 5.6 (fp32 7.9 -> 6.6; 7.2 with candidates
+// scored by every wave).  2 to 8 are the same there; with one row of each group
+// twice 2 and 4 33 us, 6 35, 8 38.
+constexpr int kFewOpen = 4;
 constexpr float kNoSim = -1e30f;       // no similarity yet (finite: its low bits carry a code too)
 
 // Nearest centroid of one (token, group) against the codebook rows cbg[c * GG ..]
@@ -502,11 +510,55 @@ __device__ __forceinline__ void encode_tokens(const EncodeArgs& a, const KeyRegs
   const float unit = K32 ? 256.f : r;
   // a zero key scores 0 on every finite row: the first code wins (8,192 x 8
   // tokens at three tiers, every fp16 key zero: 66 -> 21 us; every eighth: 66
-  // -> 25; fp32: 75 -> 29 and 74 -> 34; none: 25 and 36)
+  // -> 23; fp32: 75 -> 29 and 74 -> 31; none: 22 and 33)
   const bool open = live && (((bad_pages >> j) & 1u) || (!zero && (!(a0 - c0 > kGapSlack * unit + 1e-30f) ||
                                                                    !(a0 > 0.1f * kNoSim) || (K32 && r < kMinNorm))));
   const uint32_t best = __builtin_bit_cast(uint32_t, a0);
   code = live ? (open ? (int)(best < kOpenCode ? kOpenCode : best) : zero ? 0 : code) : 0;
+}
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), lane));
+}
+
+// Value of the lane N places along in each row of 16 (DPP row_ror).
+template <int N>
+__device__ __forceinline__ float row_ror(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x120 + N, 0xF, 0xF, true));
+}
+
+// Code of one (token, group) by the whole wave, a lane per code (lanes past C
+// repeat the last): its value `lane mod GG` is x, its norm r, its codebook's
+// rows at cb.  Same operations and the same winner as encode_group.
+template <int GG>
+__device__ __forceinline__ int score_alone(const float* cb, int C, float x, float r, bool fp16_in, int ord, int lane) {
+  float w[GG];
+#pragma unroll
+  for (int q = 0; q < GG / 4; ++q) {
+    const float4 v = *reinterpret_cast<const float4*>(cb + GG * min(lane, C - 1) + 4 * q);
+    w[4 * q] = v.x; w[4 * q + 1] = v.y; w[4 * q + 2] = v.z; w[4 * q + 3] = v.w;
+  }
+  float d, dir[GG];
+  group_directions<1>(&x, __fadd_rn(r, 1e-8f), fp16_in, &d);
+#pragma unroll
+  for (int i = 0; i < GG; ++i) dir[i] = lane_value(d, i);
+  float sim;
+  if (ord * GG * C < 400) {
+    sim = code_sim<GG, true>(dir, w);
+  } else if (GG == 16 && ord == 1) {
+    if constexpr (GG == 16) sim = code_sim_m1(dir, w);
+  } else {
+    sim = code_sim<GG, false>(dir, w);
+  }
+  // the first maximum: NaNs are passed over, but nothing exceeds a first NaN
+  const float first = lane_value(sim, 0);
+  if (!(first == first)) return 0;
+  float mx = rows_max(sim);
+  mx = fmaxf(mx, row_ror<8>(mx));
+  mx = fmaxf(mx, row_ror<4>(mx));
+  mx = fmaxf(mx, row_ror<2>(mx));
+  mx = fmaxf(mx, row_ror<1>(mx));
+  return (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(sim == mx));
 }
 
 // The wave's (token, group)s that encode_tokens left open, scored exactly.
@@ -518,6 +570,33 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
   asm volatile("" : "+v"(lane));
   const int j = lane >> 4, t = lane & 15;
   const TokenMeta mt = reload_token<CODES>(a, pc, t);
+  // a few: one after the other, their metadata and keys as scalars
+  uint64_t few = __builtin_amdgcn_ballot_w64(open);
+  if (__builtin_popcountll(few) <= kFewOpen) {
+    for (; few; few &= few - 1) {
+      const int lead = (int)__builtin_ctzll(few);
+      const int tid = uniform(__builtin_amdgcn_readlane(tid_l, lead)), h = uniform(__builtin_amdgcn_readlane(head_l, lead));
+      const int ord = uniform(__builtin_amdgcn_readlane(mt.ord, lead));
+      const float r1 = lane_value(r, lead);
+      const int64_t row = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(mt.row >> 32), lead) << 32 |
+                                    (uint32_t)__builtin_amdgcn_readlane((int)mt.row, lead));
+      const uint8_t* key = xs + PB * (lead >> 4);
+      int c;
+      if (tid != 3) {
+        const float* rows = a.cb[tid] + ((int64_t)h * (DH / 16) + w) * tier_C(tid) * 16;
+        const float x = K32 ? static_cast<const float*>(a.k)[row * DH + 16 * w + t]
+                            : (float)reinterpret_cast<const _Float16*>(key + 32 * (lead & 15))[t];
+        c = score_alone<16>(rows, tier_C(tid), x, r1, !K32, ord, lane);
+      } else {
+        const float* rows = a.cb[3] + ((int64_t)h * (DH / 32) + w) * 8 * 32;
+        const float x = K32 ? static_cast<const float*>(a.k)[row * DH + 32 * w + (lane & 31)]
+                            : (float)reinterpret_cast<const _Float16*>(key + 64 * (lead & 15))[lane & 31];
+        c = score_alone<32>(rows, 8, x, r1, !K32, ord, lane);
+      }
+      if (lane == lead) code = c;
+    }
+    return;
+  }
   // a gap within the slack: the page's similarities again, for the codes
   // within it of the best (whose bits `code` holds); then all pages' tokens
   // together, codes of repeated rows without scoring.  A wave in 30 comes here
@@ -528,8 +607,8 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
   // once (fp32 keys against rows with a twin one ulp away: 73 -> 60 us).  8,192
   // x 8 fp16 tokens at three tiers, with one row of each group twice / every
   // row / every row four times: 33 / 39 / 43 us (every lane scoring its
-  // candidates: 41 / 42 / 45), fp32 keys 44 / 49 / 53 (52 / 52 / 54); without
-  // ties 25 and 36.  (Tier 3 by candidates too was slower: 40 and 48 for 36
+  // candidates: 41 / 42 / 45), fp32 keys 45 / 49 / 53 (52 / 52 / 54); without
+  // ties 22 and 33.  (Tier 3 by candidates too was slower: 40 and 48 for 36
   // and 41.)
   uint64_t mk = 0;                                       // this lane's token: codes within the slack
   const float thr = __builtin_bit_cast(float, code) - (kGapSlack * (K32 ? 256.f : r) + 1e-30f);
@@ -609,11 +688,11 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
 // and codebook) and about 650 VALU instructions per wave, some 10 us under
 // load, so the rate is the workgroups resident: three per CU at 80 VGPRs and
 // 29 KB of LDS (fp32 keys 52.5 KB; at dh 64 57 KB and two.  With an area of
-// their own for the page images it was two at dh 128 too: 43 us for 36 below).
+// their own for the page images it was two at dh 128 too, a fifth slower).
 // Eight waves per SIMD (64 VGPRs) spill: 462 us against 315 for the
 // 98,000-token batch below.  Measured (per launch): 16 prompts of 500..12,000
 // tokens 254 -> 188 us (3.7 TB/s of traffic), 8,192 tokens 26.7 -> 22.8, the
-// same tokens' codes at three tiers 43.4 -> 26.3, of fp32 keys 52 -> 36.
+// same tokens' codes at three tiers 43.4 -> 23.0, of fp32 keys 52 -> 33.
 template <int DH, bool K32, bool CODES>
 __global__ __launch_bounds__(kEncWaves * 64) __attribute__((amdgpu_waves_per_eu(6, 6))) void encode_pages_kernel(EncodeArgs a) {
   using L = EncodeLds<DH, K32>;

@@ -348,3 +348,31 @@ def test_encode_ties_of_negative_and_zero_similarities(gpu, fp32):
     r, c, cpu = _codes_and_radii(gpu, rng, K, tier_of, cbs, H, L, dh)
     assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
     assert (r.view(np.uint32) == cpu["r"].view(np.uint32)).all()
+
+
+@pytest.mark.parametrize("fp32", [False, True])
+@pytest.mark.parametrize("dh,tier", [(128, 1), (128, 2), (128, 3), (64, 1), (64, 2), (64, 3)])
+def test_encode_few_open_codes_of_a_wave(gpu, dh, tier, fp32):
+    # runs of 64 tokens (a wave's) of one tier with 0..6 codes that the ranking
+    # leaves open: whole and near ties, NaN, infinite and tiny keys; the last
+    # page holds one token (torch's M = 1 and small orders)
+    rng = np.random.default_rng(100 * tier + dh)
+    H, L = 3, 64 * 7 + 1
+    cbs = synth.make_codebooks(rng, H, dh, [1, 2, 3])
+    cb = cbs[tier]
+    G, C, g = cb.shape[1:]
+    cb[:, :, C - 1] = cb[:, :, 1]
+    K = np.zeros((H, L, dh), np.float64)
+    for h in range(H):
+        for t in range(L):
+            x = cb[h, np.arange(G), rng.integers(2, C - 1, G)] + 0.02 * rng.standard_normal((G, g))
+            if t % 64 % 10 < (t // 64 if t < L - 1 else 10) and t % 64 < 10:
+                a, b = rng.integers(2, C - 1, 2)
+                x = (cb[h, :, 1], cb[h, :, a] + cb[h, :, b] * (1 - 10.0 ** rng.uniform(-7, -4)),
+                     1e-20 * x, np.where(rng.random(x.shape) < 0.1, np.inf, x), np.where(rng.random(x.shape) < 0.05, np.nan, x),
+                     -cb[h, :, 1])[(t + h) % 6]
+            K[h, t] = np.asarray(x).reshape(-1)
+    K = K.astype(np.float32 if fp32 else np.float16)
+    log(f"few open codes dh={dh} tier={tier} fp32={fp32}")
+    _, c, cpu = _codes_and_radii(gpu, rng, K, [np.full(L, tier, np.int32) for _ in range(H)], cbs, H, L, dh)
+    assert (c == cpu["codes"]).all(), f"{int((c != cpu['codes']).sum())} codes differ"
