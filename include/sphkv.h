@@ -611,9 +611,9 @@ int sphkv_plan_pages_fill(const uint8_t* tier_of, int64_t tier_stride, const int
  * sphkv_work_pool_rows_per_item: rows per item of a pool's own list: the
  * above at one slot per CU, or the smallest r >= 64 whose items run in three
  * rounds (r >= 64 of the above with more than 3 * num_cus ranges), whichever
- * bounds the step's time lower: an item costs its CU about 30 rows more than
- * it holds, and the step ends at most its longest item after the CUs' mean
- * load.  Returns r >= 8, or a negative SPHKV_E* code.
+ * is estimated sooner: an item costs its CU about 30 rows more than it holds,
+ * and the step ends about half of its longest item after the CUs' mean load
+ * (one round: with its longest item).  Returns r >= 8, or a negative SPHKV_E* code.
  *
  * sphkv_work_fill: work int32 [n, 4] = (sh, first_row, end_row, stride) with
  * n = sum_i max(1, ceil(len_i / rows_per_item)) (capacity max_items), and

@@ -71,12 +71,12 @@ def auto_rows_per_item(row_start: np.ndarray, num_cus: int, slots_per_cu: int = 
 def pool_rows_per_item(row_start: np.ndarray, num_cus: int) -> int:
     """Rows per work item of a pool's own list (library routine
     sphkv_work_pool_rows_per_item): auto_rows_per_item's items, or fewer and
-    larger ones that run in three rounds, whichever bounds the step lower.  An
+    larger ones that run in three rounds, whichever is estimated sooner.  An
     item costs its CU a prologue and a merge worth 30 rows, so short contexts
     want few items: 64 sequences of 150..2100 tokens (512 ranges) take 59.1 us
     per step as 1,264 items, 52.8 as 768, 54.0 as 512 and 58.1 as 816 (a fourth
     round); 64 of 300..600 40.7 as 1,224, 27.9 as 512; 26 of 200..16,000 (208
-    ranges) 130.8 as 256, 118.0 as 464.  Where the prologues count for little,
+    ranges) 131.7 as 256, 111.7 as 768.  Where the prologues count for little,
     smaller items balance better (64 of 2K..32K: 523 us as 1,264 items, 551 as
     760), and near three ranges per CU three rounds leave none to split a long
     sequence with."""

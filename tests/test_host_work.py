@@ -182,12 +182,14 @@ def test_pool_rows_per_item_is_no_worse_than_one_item_per_cu(seed):
 
 
 def test_pool_rows_per_item_of_uneven_batches():
-    # 64 sequences of 150..2100 and of 2K..32K tokens, 26 of 200..16,000, 16
-    # of 500..12,000 and one of 32K, 8 kv heads each
+    # batches timed with both lists (sequences x their range of tokens, 8 kv
+    # heads each): the items of the faster one
     def lens(n, lo, hi):
         at = [lo + int((hi - lo) * ((i * 0.6180339887498949 + 0.5) % 1.0)) for i in range(n)]
         return np.repeat([-(-t // 16) for t in at], 8)
-    for args, items in (((64, 150, 2100), 768), ((64, 2048, 32768), 1272), ((26, 200, 16000), 768), ((16, 500, 12000), 256)):
+    for args, items in (((64, 150, 2100), 768), ((64, 2048, 32768), 1272), ((26, 200, 16000), 768), ((16, 500, 12000), 256),
+                        ((24, 1356, 8957), 768), ((21, 6896, 16608), 768), ((30, 300, 16000), 768), ((40, 512, 4096), 768),
+                        ((18, 1150, 1400), 256), ((16, 2000, 9000), 256)):
         x = lens(*args)
         rs = np.concatenate([[0], np.cumsum(x)]).astype(np.int64)
         assert _items(x, ops.pool_rows_per_item(rs, 256)) == items, args
