@@ -39,26 +39,25 @@ def omega_ema(m_q: torch.Tensor, l_q: torch.Tensor, omega_prev: torch.Tensor, nu
     per-page attention mass (spherical_kv_pipeline.py:970-987)."""
     _view_ok(m_q, "m_q")
     _view_ok(l_q, "l_q")
-    nq = int(num_kv) * int(kv_groups)
-    if tuple(m_q.shape) != (nq, int(max_blocks)) or m_q.shape != l_q.shape or m_q.stride() != l_q.stride():
+    num_kv, kv_groups, max_blocks = int(num_kv), int(kv_groups), int(max_blocks)
+    nq, shape, strides = num_kv * kv_groups, m_q.shape, m_q.stride()
+    if tuple(shape) != (nq, max_blocks) or shape != l_q.shape or strides != l_q.stride():
         raise ValueError(f"m_q and l_q must be [{nq}, {max_blocks}] views with equal strides")
     omega_prev = omega_prev.contiguous()
-    if omega_prev.dtype != torch.float32 or tuple(omega_prev.shape) != (int(num_kv), int(max_blocks)):
+    if omega_prev.dtype != torch.float32 or tuple(omega_prev.shape) != (num_kv, max_blocks):
         raise ValueError(f"omega_prev must be fp32 [{num_kv}, {max_blocks}]")
     if out is None:
         out = torch.empty_like(omega_prev)
     elif out.dtype != torch.float32 or not out.is_contiguous() or out.shape != omega_prev.shape:
         raise ValueError("out must be a contiguous fp32 tensor shaped like omega_prev")
-    need = _workspace_bytes(int(num_kv), int(kv_groups), int(max_blocks), m_q.stride(1))
+    need = _workspace_bytes(num_kv, kv_groups, max_blocks, strides[1])
     if need <= 0:                                        # one kernel (and, for bad sizes, the call's own error)
-        rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1), omega_prev.data_ptr(),
-                                  out.data_ptr(), int(num_kv), int(kv_groups), int(max_blocks), float(ema_beta),
-                                  sphkv_lib.current_stream())
+        rc = _lib.sphkv_omega_ema(m_q.data_ptr(), l_q.data_ptr(), *strides, omega_prev.data_ptr(), out.data_ptr(),
+                                  num_kv, kv_groups, max_blocks, float(ema_beta), sphkv_lib.current_stream())
     else:                                                # long tables: two kernels over scratch of this call's stream
         ws = m_q.new_empty(need // 4)
-        rc = _lib.sphkv_omega_ema_ws(m_q.data_ptr(), l_q.data_ptr(), m_q.stride(0), m_q.stride(1),
-                                     omega_prev.data_ptr(), out.data_ptr(), int(num_kv), int(kv_groups),
-                                     int(max_blocks), float(ema_beta), ws.data_ptr(), need,
+        rc = _lib.sphkv_omega_ema_ws(m_q.data_ptr(), l_q.data_ptr(), *strides, omega_prev.data_ptr(), out.data_ptr(),
+                                     num_kv, kv_groups, max_blocks, float(ema_beta), ws.data_ptr(), need,
                                      sphkv_lib.current_stream())
     check(rc, "omega_ema")
     return out
