@@ -691,7 +691,7 @@ __device__ __forceinline__ void score_open(const EncodeArgs& a, const uint8_t* x
 // their own for the page images it was two at dh 128 too, a fifth slower).
 // Eight waves per SIMD (64 VGPRs) spill: 462 us against 315 for the
 // 98,000-token batch below.  Measured (per launch): 16 prompts of 500..12,000
-// tokens 254 -> 188 us (3.7 TB/s of traffic), 8,192 tokens 26.7 -> 22.8, the
+// tokens 254 -> 180 us (3.9 TB/s of traffic), 8,192 tokens 26.7 -> 19.7, the
 // same tokens' codes at three tiers 43.4 -> 23.0, of fp32 keys 52 -> 33.
 template <int DH, bool K32, bool CODES>
 __global__ __launch_bounds__(kEncWaves * 64) __attribute__((amdgpu_waves_per_eu(6, 6))) void encode_pages_kernel(EncodeArgs a) {
